@@ -21,7 +21,8 @@ BUILD_DIR = PACKAGE_DIR / "_build"
 LIB_PATH = PACKAGE_DIR / "mi355x_pisa" / "libpisa_hip.so"
 ARCH = "gfx950"
 
-SOURCES = ("api.hip", "stats.hip", "route.hip", "attention.hip", "attention_dense.hip", "fixed_block.hip", "layout.hip")
+SOURCES = ("api.hip", "stats.hip", "route.hip", "attention.hip", "attention_dense.hip", "attention_d64.hip",
+           "fixed_block.hip", "layout.hip")
 
 COMMON_FLAGS = [
     f"--offload-arch={ARCH}",

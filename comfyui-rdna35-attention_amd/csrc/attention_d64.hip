@@ -1,0 +1,426 @@
+// Attention at head dims up to 64 (padded width 64): dense, and the PISA list
+// of selected blocks and centroids with the merge and first-order correction
+// (attention.hip describes the computation; the operand tables, the transposed
+// scores and the lazy softmax are the same).
+#include "attention_softmax.hpp"
+#include "kernels.hpp"
+
+namespace pisa {
+
+namespace {
+
+constexpr int kD = 64;
+constexpr int KT = kD / 16;  // 16-deep k-steps of the score products
+constexpr int MD = kD / 32;  // 32-dim output tiles
+constexpr int NT = 2;        // 32-row query tiles of a 64-row block
+constexpr int kBlockBytes = kD * kBlock * 2;
+constexpr int kRawFlags = 0x00020000;  // untyped 32-bit buffer data format
+
+// Two waves per SIMD (256 registers each).  What bounds the loop, from
+// register-only loops of its instruction mix (one MI355X, random operands):
+// per 32-key half chunk the 16 MFMAs hold the matrix core 512 cycles and the
+// vector issue port about 15 cycles each, the 94 ordinary softmax instructions
+// 3.9 and the 32 exponentials 8 each, 863 cycles in all (measured 858 with two
+// waves, 889 with one), and each 1 KB operand fragment loaded adds about 10
+// cycles with two waves per SIMD and 22 with one: 490 ns per half chunk with
+// all operands from L2, at the 1.84-2.0 GHz that power leaves (fewer vector
+// instructions lower the cycles and the clock together).  The kernel takes
+// 540-580 ns; the one-wave kernel before it 555-610.  256 registers hold one
+// set of key and one of value fragments, each reloaded for the next half chunk
+// as soon as its products are issued: the other wave covers the latency.
+//
+// W waves share one query block, each walking a contiguous part of its chunk
+// list for all 64 query rows, and merge through LDS (fixed order, so the
+// result is reproducible): per column the running maxima, then the parts of O
+// scaled to the common maximum and summed by output units.  Every key and value
+// byte is still loaded once per query block.  launch_t chooses W.
+template <typename T, bool SPARSE, bool TAIL, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uint32_t* __restrict__ selmask) {
+    typedef typename Elem<T>::vec8 vec8;
+    const int lane = threadIdx.x & 63;
+    const int wave = W > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
+    const int half = lane >> 5;
+    const int col = lane & 31;
+    const float c = a.scale_log2;
+    const int work = xcd_remap(blockIdx.x, gridDim.x);
+    const int bh = work / a.q_blocks;
+    const int qb = work - bh * a.q_blocks;
+
+    // ---- query rows: qreg[nt][t] = Q[row 32nt + col][16t + 8half .. +7], zero past the real head dim
+    vec8 qreg[NT][KT];
+    const int qbase = a.qmap.block_base(qb);
+    int q_off[NT];
+    {
+        const char* q_head = a.q.data + a.q.row(bh, 0) * (int64_t)sizeof(T) + half * 16;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            q_off[nt] = a.qmap.intra_offset(32 * nt + col);
+            const int tok = min(qbase + q_off[nt], a.q_tokens - 1);  // rows past the end are never stored
+            const char* p = q_head + (int64_t)tok * a.q.st * (int64_t)sizeof(T);
+#pragma unroll
+            for (int t = 0; t < KT; ++t) {
+                if (t * 16 + half * 8 < a.head_dim) {
+                    qreg[nt][t] = load8<vec8>(p + t * 32);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) qreg[nt][t][e] = T(0.0f);
+                }
+            }
+        }
+    }
+
+    f32x16 o[MD][NT];
+#pragma unroll
+    for (int md = 0; md < MD; ++md)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) o[md][nt][v] = 0.0f;
+    float nm[NT], mth[NT], l[NT], lt[NT];  // running max as -m and m + kLazyRescale (rescale_to)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        nm[nt] = 0.0f;
+        mth[nt] = -__builtin_inff();
+        l[nt] = 0.0f;
+        lt[nt] = 0.0f;
+    }
+
+    // ---- chunk list: [0, n_exact) exact blocks, [n_exact, n_chunks) centroid
+    // chunks; this wave's part is [lo, hi), never empty (W <= n_chunks)
+    const int n_exact = SPARSE ? a.exact : a.kv_blocks;
+    const int n_chunks = n_exact + (TAIL ? a.npad / kBlock : 0);
+    const int lo = wave * n_chunks / W;
+    const int hi = (wave + 1) * n_chunks / W;
+    const int32_t* my_idx = SPARSE ? sel + ((int64_t)bh * a.q_blocks + qb) * a.exact : nullptr;
+    const uint32_t* my_mask = TAIL ? selmask + ((int64_t)bh * a.q_blocks + qb) * a.mask_words : nullptr;
+    // packed tables of this head as buffer resources (reads past a table return zero)
+    const int tab_bytes = a.kv_blocks * kBlockBytes;
+    const __amdgpu_buffer_rsrc_t kp_rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(a.kp + (int64_t)bh * a.kv_blocks * kBlockBytes), (short)0, tab_bytes, kRawFlags);
+    const __amdgpu_buffer_rsrc_t vp_rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(a.vp + (int64_t)bh * a.kv_blocks * kBlockBytes), (short)0, tab_bytes, kRawFlags);
+    const int cen_bytes = TAIL ? a.npad * kD * 2 : 0;
+    const __amdgpu_buffer_rsrc_t kc_rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(TAIL ? a.kbar + (int64_t)bh * a.npad * kD * 2 : a.kp), (short)0, cen_bytes, kRawFlags);
+    const __amdgpu_buffer_rsrc_t vc_rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(TAIL ? a.vbar_t + (int64_t)bh * a.npad * kD * 2 : a.vp), (short)0, cen_bytes, kRawFlags);
+    const int lane_off = lane * 16;
+
+    auto is_tail = [&](int x) { return TAIL && min(x, n_chunks - 1) >= n_exact; };
+    auto table_row = [&](int x) -> int {  // block id, or centroid chunk id; past the list, its last chunk again
+        x = min(x, n_chunks - 1);
+        if (TAIL && x >= n_exact) return x - n_exact;
+        return SPARSE ? my_idx[x] : x;
+    };
+    auto ld_frag = [&](const __amdgpu_buffer_rsrc_t& rs, int off, int frag) -> vec8 {
+        const int soff = __builtin_amdgcn_readfirstlane(off + (frag >> 2) * 4096);
+        return __builtin_bit_cast(vec8,
+                                  __builtin_amdgcn_raw_buffer_load_b128(rs, lane_off + (frag & 3) * 1024, soff, 0));
+    };
+
+    vec8 kf[KT];     // key fragments of the half chunk scored next
+    vec8 vf[MD][2];  // value fragments of the half chunk multiplied next
+    auto load_k = [&](bool tail, int row, int mt) {
+#pragma unroll
+        for (int t = 0; t < KT; ++t) kf[t] = ld_frag(tail ? kc_rs : kp_rs, row * kBlockBytes, mt * KT + t);
+    };
+    auto load_v = [&](bool tail, int row, int mt) {
+#pragma unroll
+        for (int md = 0; md < MD; ++md)
+#pragma unroll
+            for (int ss = 0; ss < 2; ++ss)
+                vf[md][ss] = ld_frag(tail ? vc_rs : vp_rs, row * kBlockBytes, md * 4 + 2 * mt + ss);
+    };
+    // Centroid chunks get their score bias (log2 of the block's length over c,
+    // -inf for selected blocks and padding) from one more MFMA per query tile:
+    // lane (0, col) of the A operand holds centroid col's bias as bf16 parts,
+    // the B operand ones in those slots.  bf16 for both input types (bias / c
+    // can exceed fp16's range at small softmax scales); three parts carry the
+    // fp32 value exactly.
+    bf16x8 ones_frag;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ones_frag[e] = (bf16_t)((half == 0 && e < 3) ? 1.0f : 0.0f);
+    auto bias_frag = [&](int row, int mt) -> bf16x8 {
+        bf16x8 f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = (bf16_t)0.0f;
+        const uint32_t word = (2 * row + mt < a.mask_words) ? my_mask[2 * row + mt] : 0u;
+        const int j = row * kBlock + mt * 32 + col;
+        const bool dead = ((word >> col) & 1u) != 0u || j >= a.centroids;
+        const float b = (j == a.centroids - 1 ? a.last_len_log2 : 6.0f) * a.inv_scale_log2;
+        const bf16_t b0 = (bf16_t)b;
+        const float r1 = b - (float)b0;
+        const bf16_t b1 = (bf16_t)r1;
+        if (half == 0) {
+            f[0] = dead ? (bf16_t)(-__builtin_inff()) : b0;
+            f[1] = dead ? (bf16_t)0.0f : b1;
+            f[2] = dead ? (bf16_t)0.0f : (bf16_t)(r1 - (float)b1);
+        }
+        return f;
+    };
+    // scores of half mt of the chunk in table row `row` (its key fragments are in kf)
+    auto scores = [&](f32x16 (&s)[NT], bool tail, int row, int mt) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) s[nt][v] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) s[nt] = mfma32(kf[t], qreg[nt][t], s[nt]);
+        if (TAIL && tail) {
+            const bf16x8 b = bias_frag(row, mt);
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) s[nt] = mfma32(b, ones_frag, s[nt]);
+        }
+    };
+    auto pv = [&](const vec8 (&pf)[NT][2]) {
+#pragma unroll
+        for (int ss = 0; ss < 2; ++ss)
+#pragma unroll
+            for (int md = 0; md < MD; ++md)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) o[md][nt] = mfma32(vf[md][ss], pf[nt][ss], o[md][nt]);
+    };
+    // column maxima and running-max update of half mt of a chunk; `plain`: an
+    // exact full block, else a short last key block is masked first
+    auto check = [&](f32x16 (&s)[NT], bool tail, int row, int mt, bool plain) {
+        if (!plain && !tail && (row + 1) * kBlock > a.kv_tokens) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                if (row * kBlock + mt * 32 + 8 * (v >> 2) + 4 * half + (v & 3) >= a.kv_tokens)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt) s[nt][v] = -__builtin_inff();
+        }
+        float mx[NT];
+        half_max<NT>(s, c, mx);
+        rescale_to<NT, MD>(mx, true, nm, mth, l, lt, o);
+    };
+
+    f32x16 sa[NT], sb[NT];  // scores of the first / second half of the current chunk
+    int row0 = table_row(lo), row1 = table_row(lo + 1);
+    load_k(is_tail(lo), row0, 0);
+    load_v(is_tail(lo), row0, 0);
+    scores(sa, is_tail(lo), row0, 0);
+    load_k(is_tail(lo), row0, 1);
+    check(sa, is_tail(lo), row0, 0, false);
+    // One chunk: its first half's softmax and PV product beside the scores of
+    // its second half, then the second half's beside the scores of the next
+    // chunk.  `last` (no next chunk) and `plain` (this chunk and the next are
+    // exact full blocks) are constants of each inlined copy.
+    auto chunk_step = [&](int cc, bool last, bool plain) __attribute__((always_inline)) {
+        const int row2 = (plain && !SPARSE) ? cc + 2 : table_row(cc + 2);
+        const bool t0 = !plain && is_tail(cc), t1 = !plain && !last && is_tail(cc + 1);
+        vec8 pf[NT][2];
+        scores(sb, t0, row0, 1);
+        if (!last) load_k(t1, row1, 0);
+        probs_half<T, NT>(sa, c, nm, l, lt, t0, pf);
+        pv(pf);
+        load_v(t0, row0, 1);
+        check(sb, t0, row0, 1, plain);
+
+        if (!last) {
+            scores(sa, t1, row1, 0);
+            load_k(t1, row1, 1);
+        }
+        probs_half<T, NT>(sb, c, nm, l, lt, t0, pf);
+        pv(pf);
+        if (!last) {
+            load_v(t1, row1, 0);
+            check(sa, t1, row1, 0, plain);
+        }
+        row0 = row1;
+        row1 = row2;
+    };
+    // the selection is ascending, so only the last exact chunk can be short
+    int cc = lo;
+    for (; cc + 3 <= n_exact && cc + 1 < hi; ++cc) chunk_step(cc, false, true);
+    for (; cc + 1 < hi; ++cc) chunk_step(cc, false, false);
+    chunk_step(cc, true, false);
+
+    // ---- merge of the W parts, first-order correction, store
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        l[nt] = add_xor32(l[nt]);
+        lt[nt] = add_xor32(lt[nt]);
+    }
+    constexpr int kUnits = MD * NT * 2;  // (tile, pair of 4-row groups) output units, kUnits / W per wave
+    __shared__ __attribute__((aligned(16))) float parts[W > 1 ? W * MD * NT * 16 * 64 : 4];
+    __shared__ float stat[W > 1 ? W : 1][3][kBlock];
+    if constexpr (W > 1) {
+        float m[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            m[nt] = mth[nt] == -__builtin_inff() ? -__builtin_inff() : -nm[nt];
+            if (half == 0) {
+                stat[wave][0][32 * nt + col] = m[nt];
+                stat[wave][1][32 * nt + col] = l[nt];
+                stat[wave][2][32 * nt + col] = lt[nt];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            float top = -__builtin_inff();
+#pragma unroll
+            for (int w = 0; w < W; ++w) top = fmaxf(top, stat[w][0][32 * nt + col]);
+            auto factor = [&](float mw) { return mw == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(mw - top); };
+            l[nt] = 0.0f;
+            lt[nt] = 0.0f;
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const float f = factor(stat[w][0][32 * nt + col]);
+                l[nt] += stat[w][1][32 * nt + col] * f;
+                lt[nt] += stat[w][2][32 * nt + col] * f;
+            }
+            const float f = factor(m[nt]);
+#pragma unroll
+            for (int md = 0; md < MD; ++md)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    f32x4 x;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[e] = o[md][nt][4 * g + e] * f;
+                    *reinterpret_cast<f32x4*>(&parts[((((wave * MD + md) * NT + nt) * 4 + g) * 64 + lane) * 4]) = x;
+                }
+        }
+        __syncthreads();
+    }
+    const bool first_order = TAIL && a.ht != nullptr;
+    const __amdgpu_buffer_rsrc_t ht_rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(first_order ? a.ht + (int64_t)bh * kD * kD * 2 : a.kp), (short)0, first_order ? kD * kD * 2 : 0,
+        kRawFlags);
+    typedef T vec4 __attribute__((ext_vector_type(4)));
+    // 16-byte stores when every output row start is 16-byte aligned (8-byte ones otherwise)
+    const bool st16 = (reinterpret_cast<uintptr_t>(a.o.data) % 16 == 0) &&
+                      ((a.o.sb | a.o.sh | a.o.st) * (int64_t)sizeof(T)) % 16 == 0;
+#pragma unroll
+    for (int u = 0; u < kUnits / W; ++u) {
+        // W = 1: tile and pair are constants and the accumulators stay in registers
+        const int unit = wave * (kUnits / W) + u;
+        const int p = unit & 1, nt = (unit >> 1) & 1, md = unit >> 2;
+        const bool second = nt != 0;
+        float x[8];
+        if constexpr (W > 1) {
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int w = 0; w < W; ++w)
+                    sum += *reinterpret_cast<const f32x4*>(
+                        &parts[((((w * MD + md) * NT + nt) * 4 + 2 * p + g) * 64 + lane) * 4]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[4 * g + e] = sum[e];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = o[u >> 2][(u >> 1) & 1][8 * (u & 1) + e];
+        }
+        const float lf = second ? l[1] : l[0];
+        const float inv = 1.0f / lf;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] *= inv;
+        if (first_order) {
+            // rows 32md .. of the packed D x D matrix (kfrag_elem) times the query tile
+            f32x16 corr;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) corr[v] = 0.0f;
+#pragma unroll
+            for (int t = 0; t < KT; ++t)
+                corr = mfma32(ld_frag(ht_rs, md * KT * 1024, t), second ? qreg[1][t] : qreg[0][t], corr);
+            const float wa = (second ? lt[1] : lt[0]) * inv * a.corr_scale;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] += (p ? corr[8 + e] : corr[e]) * wa;
+        }
+        const int tok = qbase + (second ? q_off[1] : q_off[0]);
+        if (tok >= a.q_tokens) continue;  // lanes l and l + 32 (one query) take the same branch
+        char* dst = a.o.data + a.o.row(bh, tok) * (int64_t)sizeof(T);
+        u32x2 w4[2];  // w4[g]: dims 32md + 8(2p + g) + 4half ..
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            vec4 out;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[e] = from_f32<T>(x[4 * g + e]);
+            w4[g] = __builtin_bit_cast(u32x2, out);
+        }
+        if (st16) {
+            // one lane-half swap per dword leaves lanes 0-31 with dims 8(2p) .. +7 and
+            // lanes 32-63 with dims 8(2p + 1) .. +7 of the tile
+            u32x4 x16;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const auto r = __builtin_amdgcn_permlane32_swap(w4[0][j], w4[1][j], false, false);
+                x16[j] = r[0];
+                x16[2 + j] = r[1];
+            }
+            const int d = md * 32 + 8 * (2 * p + half);
+            if (d < a.head_dim) *reinterpret_cast<u32x4*>(dst + d * sizeof(T)) = x16;
+        } else {
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                const int d = md * 32 + 8 * (2 * p + g) + 4 * half;
+                if (d < a.head_dim) *reinterpret_cast<u32x2*>(dst + d * sizeof(T)) = w4[g];
+            }
+        }
+    }
+}
+
+// Waves per query block: the W with the smallest estimate of
+//     rounds of the SIMDs x (chunks of one wave + the chunk times a merge costs),
+// which follows the measured times (1280 blocks of 64 chunks, [2,10,4096,64]:
+// 126 / 108 / 98 / 122 us at W = 1 / 2 / 4 / 8, estimates 130 / 107 / 98 / 125;
+// 2048 such blocks: 142 / 145 / 148 / 184 us, estimates 130 / 142 / 156 / 200;
+// 128 blocks of 16 chunks: 17.7 us with one wave, under 12 with 2, 4 or 8).  A
+// grid that leaves SIMDs idle, or its last round nearly empty, is split; a full
+// one keeps one wave per block and merges nothing.  Eight waves use 134 KB of
+// LDS, one workgroup per CU, so nothing runs beside their merge.
+int waves_per_block(int64_t blocks, int n_chunks) {
+    static const int simds = [] {
+        int dev = 0, cus = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            return 0;
+        return 4 * cus;
+    }();
+    if (simds <= 0) return 1;
+    int best = 1;
+    double least = 0.0;
+    for (int w = 1; w <= 8 && w <= n_chunks; w *= 2) {
+        const double merge = w == 1 ? 1.0 : w == 8 ? 4.5 : 3.5;
+        const double cost = (double)((blocks * w + simds - 1) / simds) * ((n_chunks + w - 1) / w + merge);
+        if (w == 1 || cost < least) {
+            best = w;
+            least = cost;
+        }
+    }
+    return best;
+}
+
+template <typename T, bool SPARSE, bool TAIL>
+int launch_t(const AttnArgs& a, int bh_count, hipStream_t stream) {
+    const int blocks = bh_count * a.q_blocks;
+    const int n_chunks = (SPARSE ? a.exact : a.kv_blocks) + (TAIL ? a.npad / kBlock : 0);
+    const int w = waves_per_block(blocks, n_chunks);
+#define PISA_D64(W)                                                                                              \
+    hipLaunchKernelGGL((attention_d64_kernel<T, SPARSE, TAIL, W>), dim3(blocks), dim3(64 * W), 0, stream, a, a.idx, \
+                       a.selmask)
+    if (w == 1) PISA_D64(1);
+    else if (w == 2) PISA_D64(2);
+    else if (w == 4) PISA_D64(4);
+    else PISA_D64(8);
+#undef PISA_D64
+    return pisa_host::check_launch("attention_d64_kernel");
+}
+
+}  // namespace
+
+int launch_attention_d64(int dtype, bool sparse, const AttnArgs& a, int bh_count, hipStream_t stream) {
+    if (dtype == PISA_DTYPE_BF16)
+        return sparse ? launch_t<bf16_t, true, true>(a, bh_count, stream)
+                      : launch_t<bf16_t, false, false>(a, bh_count, stream);
+    return sparse ? launch_t<f16_t, true, true>(a, bh_count, stream)
+                  : launch_t<f16_t, false, false>(a, bh_count, stream);
+}
+
+}  // namespace pisa

@@ -201,6 +201,8 @@ int launch_stats_means(int dtype, int padded, const StatsArgs& a, int bh_count, 
 // `padded` = padded_head_dim(a.head_dim); dense (sparse = tail = false) or PISA (both true).
 int launch_attention(int dtype, int padded, bool sparse, bool tail, const AttnArgs& a, int bh_count,
                      hipStream_t stream);
+// The same at padded width 64, dense or PISA (attention_d64.hip).
+int launch_attention_d64(int dtype, bool sparse, const AttnArgs& a, int bh_count, hipStream_t stream);
 // Packed key / value blocks of width `padded` (dims >= head_dim and rows >= kv_tokens are zero);
 // block j row r is token map(64 j + r).
 int launch_kv_pack(int dtype, int padded, int head_dim, const View& k, const View& v, TokenMap map, int kv_tokens,

@@ -1,0 +1,85 @@
+"""The head-dim-64 attention kernel on the MI355X at the sizes where its key split changes.
+
+One to eight waves share a query block and merge their parts of its chunk list; the split follows the number of
+query blocks and chunks, so the shapes below reach every split, ragged last blocks, lists shorter than the split
+and parts whose every score is masked.
+
+Tolerance of the dense checks: the probabilities and the output are rounded to the storage type (relative 2^-9 in
+bf16, 2^-12 in fp16, at most) and an output row is an average of the values with weights that sum to one, so an
+element is off by at most (2^-9 + 2^-9) max|v|, twice that bound being allowed.
+"""
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from helpers import assert_close, np32
+from oracle import attention as oatt
+from oracle import pisa as opisa
+
+pytestmark = pytest.mark.gpu
+UNIT = {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}
+TOL = {torch.bfloat16: 5e-2, torch.float16: 2e-2}
+
+
+@pytest.fixture(scope="module")
+def native():
+    import mi355x_pisa
+
+    return mi355x_pisa
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,q_tokens,kv_tokens,head_dim", [
+    (1, 1, 1, 64),          # one row, one key
+    (2, 65, 77, 64),        # two chunks, the second short
+    (3, 130, 1000, 40),     # eight waves, 16 chunks, short last chunk, padded dims
+    (40, 300, 1024, 64),    # 200 blocks: four waves
+    (20, 1600, 512, 64),    # 500 blocks of 8 chunks: two waves
+    (64, 1024, 130, 64),    # 1024 blocks: one wave
+    (2, 64, 449, 8),        # eight waves on eight chunks, one each
+])
+def test_dense_splits_match_oracle(native, dtype, heads, q_tokens, kv_tokens, head_dim):
+    gen = torch.Generator().manual_seed(heads * 7 + q_tokens + kv_tokens)
+    q = torch.randn((1, heads, q_tokens, head_dim), generator=gen).to(dtype)
+    k, v = (torch.randn((1, heads, kv_tokens, head_dim), generator=gen).to(dtype) for _ in range(2))
+    out = native.dense_attention(q.cuda(), k.cuda(), v.cuda(), 1 / math.sqrt(head_dim))
+    expected = oatt.dense_attention(np32(q), np32(k), np32(v))
+    atol = 4 * UNIT[dtype] * float(v.float().abs().max())
+    assert_close(np32(out), expected, atol, 0.0, f"dense {heads}x{q_tokens}x{kv_tokens} D={head_dim}")
+
+
+def test_dense_split_parts_of_very_different_scale(native):
+    """Key parts whose maxima lie far apart (and rise along the list) merge without overflow or loss."""
+    gen = torch.Generator().manual_seed(3)
+    q = torch.randn((1, 2, 64, 64), generator=gen)
+    k = torch.randn((1, 2, 512, 64), generator=gen) * torch.linspace(0.0, 12.0, 512)[:, None]
+    v = torch.randn((1, 2, 512, 64), generator=gen)
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    out = native.dense_attention(q.cuda(), k.cuda(), v.cuda(), 1.0)
+    expected = oatt.dense_attention(np32(q), np32(k), np32(v), 1.0)
+    # scores reach about 400 here: a bf16 product is exact and an fp32 sum of 64 of them is off by up to
+    # 64 * 2^-24 * 400, which moves a probability by 0.15 % beside the storage rounding
+    atol = (4 * UNIT[torch.bfloat16] + 64 * 2.0 ** -24 * 400) * float(v.float().abs().max())
+    assert_close(np32(out), expected, atol, 0.0, "rising scores")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,tokens,exact,first_order,scale", [
+    (2, 1000, 0, False, 0.125),   # centroids only: one chunk, one wave
+    (2, 500, 7, True, 0.125),     # all but one block exact, short last block
+    (1, 4100, 6, True, 0.125),    # two centroid chunks, the second nearly all padding
+    (16, 1024, 4, False, 1e-3),   # a small softmax scale: bias / scale beyond fp16's range
+])
+def test_sparse_splits_match_oracle(native, dtype, heads, tokens, exact, first_order, scale):
+    gen = torch.Generator().manual_seed(tokens + exact)
+    q, k, v = (torch.randn((1, heads, tokens, 64), generator=gen).to(dtype) for _ in range(3))
+    out, scores, idx = native.forward_with_routing(q.cuda(), k.cuda(), v.cuda(), exact, scale, mode="generic",
+                                                   first_order=first_order)
+    assert (idx.cpu().numpy() == opisa.topk_ascending(scores.cpu().numpy(), exact)).all()
+    name = "bf16" if dtype == torch.bfloat16 else "f16"
+    ref = opisa.generic_forward(*(np32(t).reshape(heads, tokens, 64) for t in (q, k, v)), exact, scale,
+                                first_order=first_order, dtype=name)
+    assert_close(np32(out).reshape(heads, tokens, 64), ref, TOL[dtype], TOL[dtype], f"sparse T={tokens}")
