@@ -1,12 +1,12 @@
 // Fixed block-diagonal attention: every 64-token block attends only to itself.
 //
-// Four kernels.  bf16/fp16 calls without a mask run fixed_block_mfma_kernel
-// (matrix cores, the reference's Triton semantics, below); fp32 calls without
-// a mask run fixed_block_f32x3_kernel (head dims 32, 64: fp32 products from
-// exact three-part bf16 splits on the bf16 matrix cores) or
-// fixed_block_f32_mfma_kernel (head dim 128: fp32 matrix cores).  Masked
-// calls and rows that are not 16-byte aligned - the calls the reference sends
-// to its eager fp32 loop - run fixed_block_kernel:
+// Four kernels.  bf16/fp16 calls run fixed_block_mfma_kernel (matrix cores;
+// without a mask the reference's Triton semantics, with one its eager fp32
+// loop's, below); fp32 calls run fixed_block_f32x3_kernel (no mask, head dims
+// 32, 64: fp32 products from exact three-part bf16 splits on the bf16 matrix
+// cores) or fixed_block_f32_mfma_kernel (head dim 128, and every masked call:
+// fp32 matrix cores).  Rows that are not 16-byte aligned run
+// fixed_block_kernel:
 //
 // One 256-thread workgroup per (block, batch*head).  The block's Q, K and V
 // (64 x D) are staged in LDS as fp32; thread (rt, kt) = (t/16, t%16) owns the
@@ -41,6 +41,71 @@ __device__ __forceinline__ float apply_mask(const MaskView& m, int64_t off, floa
         case PISA_MASK_ADD_BF16: return s + to_f32(reinterpret_cast<const bf16_t*>(m.data)[off]);
         default: return s;
     }
+}
+
+// Four mask entries of consecutive keys as loaded (MK = PISA_MASK_*), and the
+// score they turn s into.
+template <int MK> struct MaskEntries { typedef uint32_t type; };  // PISA_MASK_BOOL: a byte each
+template <> struct MaskEntries<PISA_MASK_ADD_F32> { typedef f32x4 type; };
+template <> struct MaskEntries<PISA_MASK_ADD_F16> { typedef f16_t type __attribute__((ext_vector_type(4))); };
+template <> struct MaskEntries<PISA_MASK_ADD_BF16> { typedef bf16_t type __attribute__((ext_vector_type(4))); };
+
+template <int MK>
+__device__ __forceinline__ float masked_score(float s, const typename MaskEntries<MK>::type& m, int e) {
+    if constexpr (MK == PISA_MASK_BOOL) return ((m >> (8 * e)) & 0xffu) ? s : -__builtin_inff();
+    else return s + to_f32(m[e]);
+}
+
+// Entries of keys key0 .. key0 + 3 at element offset `off` (that of key 0).
+// `wide`: one aligned load (unit key stride, a whole block); otherwise entry by
+// entry, keys past the block's `len` re-reading its last one (they are masked
+// out anyway).
+template <int MK>
+__device__ __forceinline__ typename MaskEntries<MK>::type load_mask4(const MaskView& m, int64_t off, int key0, int len,
+                                                                    bool wide) {
+    typedef typename MaskEntries<MK>::type entries;
+    if constexpr (MK == PISA_MASK_BOOL) {
+        if (wide) return *reinterpret_cast<const uint32_t*>(m.data + off + key0);
+        uint32_t x = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x |= (m.data[off + min(key0 + e, len - 1) * m.sk] ? 1u : 0u) << (8 * e);
+        return x;
+    } else {
+        typedef typename std::conditional<MK == PISA_MASK_ADD_F32, float,
+                                          typename std::conditional<MK == PISA_MASK_ADD_F16, f16_t, bf16_t>::type>::type E;
+        const E* p = reinterpret_cast<const E*>(m.data) + off;
+        if (wide) return *reinterpret_cast<const entries*>(p + key0);
+        entries x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = p[min(key0 + e, len - 1) * m.sk];
+        return x;
+    }
+}
+
+// Element offset of the entry (query start + row, key start) of head bh.
+__device__ __forceinline__ int64_t mask_row(const MaskView& m, int bh, int start, int row) {
+    const int b = bh / m.heads;
+    return b * m.sb + (bh - b * m.heads) * m.sh + (int64_t)start * (m.sq + m.sk) + row * m.sq;
+}
+
+// Whether four consecutive entries of any row and block are one aligned load.
+static bool mask_rows_wide(const MaskView& m) {
+    const int bytes = m.kind == PISA_MASK_BOOL ? 1 : m.kind == PISA_MASK_ADD_F32 ? 4 : 2;
+    return m.sk == 1 && (m.sb | m.sh | m.sq) % 4 == 0 && reinterpret_cast<uintptr_t>(m.data) % (4 * bytes) == 0;
+}
+
+// e^x for x <= 0 in fp32: 2^(x log2 e) on v_exp_f32, with the rounding error of
+// the product (an fma) and the low part of log2 e carried into a first-order
+// factor (its neglected square is below 1e-10 for x >= -100); 0 below -150
+// (e^-150 is far below the smallest fp32 value, and the product of a large
+// negative mask value overflows).  Four full-rate instructions and one
+// exponential where expf's range handling takes about a dozen (C1 9.43 ->
+// 9.06 us, same error against float64).
+__device__ __forceinline__ float exp_nonpos(float x) {
+    const float hi = x * kLog2e;
+    const float lo = fmaf(x, kLog2e, -hi) + x * 1.925963e-8f;  // log2(e) - fp32(log2(e)) = 1.925963e-8
+    const float e = __builtin_amdgcn_exp2f(hi) * fmaf(lo, 0.69314718f, 1.0f);
+    return x < -150.0f ? 0.0f : e;
 }
 
 template <typename T, int D>
@@ -165,10 +230,19 @@ __global__ __launch_bounds__(256) void fixed_block_kernel(View q, View k, View v
     }
 }
 
-// bf16 / fp16 without a mask: one wavefront per block on 32x32x16 MFMA, the
+// bf16 / fp16: one wavefront per block on 32x32x16 MFMA.  Without a mask the
 // semantics of the reference's Triton kernel (triton_kernel.py:53-100): scores
 // with fp32 accumulation, softmax in fp32, probabilities normalised and then
 // rounded to the input dtype, P @ V with fp32 accumulation, rounded output.
+// With one (MK = its PISA_MASK_* kind) those of the eager loop
+// (reference.py:179-198), whose probabilities stay fp32: the scores are the
+// same exact products, and P @ V runs on the fp32 matrix cores
+// (v_mfma_f32_32x32x2_f32: step v contracts the keys of accumulator v in the
+// two lane halves, so the probabilities feed it from the registers they are in
+// and the value operand is the element of vr below, widened).
+// [2,16,4000,64] bf16 with a [T,T] bf16 mask (66 MB): 85 us with the fp32 VALU
+// kernel, 27 us here (the matrix time is 8 us, the memory time 12); [2,24,6000,128]
+// fp16: 670 -> 110 us.
 //
 // Nothing is staged in LDS, so the occupancy is set by registers alone.  The
 // products are formed transposed as in the attention kernels (S^T = K Q^T,
@@ -180,9 +254,10 @@ __global__ __launch_bounds__(256) void fixed_block_kernel(View q, View k, View v
 // consecutive dims of a key row with one load (output tile md holds dims
 // MD*i + md of accumulator row i), one load instruction covers two whole key
 // rows, and the operand of tile md takes element md of 8 such loads.
-template <typename T, int D>
+template <typename T, int D, int MK>
 __global__ __launch_bounds__(64) void fixed_block_mfma_kernel(View q, View k, View v, OutView o, int tokens,
-                                                               int nblocks, float scale_log2, int causal) {
+                                                               int nblocks, float scale, int causal, MaskView mask,
+                                                               int mask_wide) {
     typedef typename Elem<T>::vec8 vec8;
     constexpr int KT = D / 16;  // 16-deep k-steps of the score product
     constexpr int MD = D / 32;  // output dim tiles; dims a lane reads per key row
@@ -209,6 +284,19 @@ __global__ __launch_bounds__(64) void fixed_block_mfma_kernel(View q, View k, Vi
             kf[x][t] = load8<vec8>(krow[x] + (16 * t + 8 * half) * sizeof(T));
             qf[x][t] = load8<vec8>(qrow[x] + (16 * t + 8 * half) * sizeof(T));
         }
+    typename MaskEntries<MK>::type me[MK != PISA_MASK_NONE ? 2 : 1][2][4];  // [nt][mt][e/4]: 4 keys of query (nt, col)
+    if constexpr (MK != PISA_MASK_NONE) {
+        const bool wide = mask_wide != 0 && len == 64;
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            const int64_t off = mask_row(mask, bh, start, min(32 * nt + col, len - 1));
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    me[nt][mt][g] = load_mask4<MK>(mask, off, 32 * mt + 8 * g + 4 * half, len, wide);
+        }
+    }
     // every Q and K request is issued before the first product (the
     // scheduler would otherwise issue each just before its use, one memory
     // round trip at a time), and the V requests right after the products
@@ -242,11 +330,81 @@ __global__ __launch_bounds__(64) void fixed_block_mfma_kernel(View q, View k, Vi
                 const int key = 32 * mt + 16 * ss + 4 * half + 8 * (e >> 2) + (e & 3);
                 vr[mt][ss][e] = *reinterpret_cast<const vecmd*>(at(v, key) + MD * col * sizeof(T));
             }
+    // masked: value rows past the block are zero, as in fixed_block_kernel (an
+    // infinite last row must not meet their zero probabilities)
+    if constexpr (MK != PISA_MASK_NONE) {
+        if (len < 64) {
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    if (32 * mt + 8 * (e >> 2) + 4 * half + (e & 3) >= len) vr[mt][e >> 3][e & 7] = vecmd(T(0.0f));
+        }
+    }
 
     __builtin_amdgcn_sched_barrier(0);
 
+    if constexpr (MK != PISA_MASK_NONE) {
+        // one query tile at a time: softmax in natural units, then P @ V in fp32
+        // and its store (row i of output tile md is dim MD*i + md, as below)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            const int query = 32 * nt + col;
+            float mx = -__builtin_inff();
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int key = 32 * mt + 8 * (e >> 2) + 4 * half + (e & 3);
+                    const bool dead = key >= len || (causal && key > query);
+                    const float x = masked_score<MK>(s[mt][nt][e] * scale, me[nt][mt][e >> 2], e & 3);
+                    s[mt][nt][e] = dead ? -__builtin_inff() : x;
+                    mx = fmaxf(mx, s[mt][nt][e]);
+                }
+            mx = max_xor32(mx);
+            const float m_use = mx == -__builtin_inff() ? 0.0f : mx;
+            float sum = 0.0f;
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    s[mt][nt][e] = exp_nonpos(s[mt][nt][e] - m_use);
+                    sum += s[mt][nt][e];
+                }
+            sum = add_xor32(sum);
+            const float inv = sum > 0.0f ? 1.0f / sum : __builtin_nanf("");  // all keys masked
+            f32x16 acc[MD];
+#pragma unroll
+            for (int md = 0; md < MD; ++md)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[md][e] = 0.0f;
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const float p = s[mt][nt][e] * inv;
+#pragma unroll
+                    for (int md = 0; md < MD; ++md)
+                        acc[md] = __builtin_amdgcn_mfma_f32_32x32x2f32(to_f32(vr[mt][e >> 3][e & 7][md]), p, acc[md],
+                                                                       0, 0, 0);
+                }
+            if (query < len) {
+                char* dst = o.data + o.row(bh, start + query) * (int64_t)sizeof(T);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    vecmd x;
+#pragma unroll
+                    for (int md = 0; md < MD; ++md) x[md] = from_f32<T>(acc[md][e]);
+                    *reinterpret_cast<vecmd*>(dst + MD * (8 * (e >> 2) + 4 * half + (e & 3)) * sizeof(T)) = x;
+                }
+            }
+        }
+        return;
+    }
+
     // ---- masking and the softmax of query column (nt, col), in log2 units:
     // accumulator e of tile mt is key 32mt + 8(e/4) + 4half + e%4
+    const float scale_log2 = scale * kLog2e;
     vec8 pf[2][2][2];  // [nt][mt][ss]: 8 probabilities, elements 8ss .. 8ss+7 of tile mt
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
@@ -320,10 +478,14 @@ __global__ __launch_bounds__(64) void fixed_block_mfma_kernel(View q, View k, Vi
     }
 }
 
-// fp32 without a mask: four waves per block on v_mfma_f32_16x16x4_f32 (fp32
-// operands, fp32 accumulation), the arithmetic of fixed_block_kernel above
-// (fp32 scores, softmax with expf, fp32 P @ V).  Wave w owns queries
-// 16w .. 16w+15 (a lane column c = lane % 16, lane group g = lane / 16).
+// fp32, head dim 128 or masked: four waves per block on v_mfma_f32_16x16x4_f32
+// (fp32 operands, fp32 accumulation), the arithmetic of fixed_block_kernel above
+// (fp32 scores, softmax with expf, fp32 P @ V).  Masked calls of every head dim
+// run here ([2,16,4000,64] with a [T,T] bool mask: 104 us on the VALU kernel ->
+// 45 us, [2,16,4000,128] with an fp32 one: 301 -> 81 us): the three-part splits
+// of fixed_block_f32x3_kernel turn an infinite operand into NaN, which the VALU
+// kernel does not.  Wave w owns queries 16w .. 16w+15 (a lane column c = lane %
+// 16, lane group g = lane / 16).
 //   S^T = K Q^T: k-step t = 4s + e contracts dim 16s + 4g + e in lane group g,
 //     so each lane reads its K and Q rows as float4 pieces (dims 16s + 4g ..);
 //     accumulator r of key tile n is key 16n + 4g + r of query 16w + c.
@@ -340,9 +502,10 @@ __global__ __launch_bounds__(64) void fixed_block_mfma_kernel(View q, View k, Vi
 // length are read clamped to its last row (unconditional loads, so the
 // compiler's wait counts stay partial) and get probability 0 (keys) or are not
 // stored (queries).
-template <int D>
+template <int D, int MK>
 __global__ __launch_bounds__(256) void fixed_block_f32_mfma_kernel(View q, View k, View v, OutView o, int tokens,
-                                                                   int nblocks, float scale, int causal) {
+                                                                   int nblocks, float scale, int causal,
+                                                                   MaskView mask, int mask_wide) {
     constexpr int S4 = D / 16;  // float4 pieces of a Q or K row per lane
     constexpr int VW = D / 16;  // V dims per lane per key row = output dim tiles
     constexpr int kRowF = D + 4;  // padded LDS row (floats)
@@ -365,6 +528,13 @@ __global__ __launch_bounds__(256) void fixed_block_f32_mfma_kernel(View q, View 
 #pragma unroll
         for (int s4 = 0; s4 < S4; ++s4) qv[s4] = *reinterpret_cast<const f32x4*>(qr + 16 * s4 + 4 * g);
     }
+    typename MaskEntries<MK>::type me[4];  // [n]: keys 16n + 4g .. +3 of query 16w + c
+    if constexpr (MK != PISA_MASK_NONE) {
+        const int64_t off = mask_row(mask, bh, start, min(16 * w + c, len - 1));
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+            me[n] = load_mask4<MK>(mask, off, 16 * n + 4 * g, len, mask_wide != 0 && len == 64);
+    }
     float vv[4][4][VW];
     {
         // staging: lane l of wave w loads dims D/4 (l%4) .. of row 16w + l/4 of K and V
@@ -382,7 +552,10 @@ __global__ __launch_bounds__(256) void fixed_block_f32_mfma_kernel(View q, View 
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             *reinterpret_cast<f32x4*>(&ks[row * kRowF + d0 + 4 * p]) = xk[p];
-            *reinterpret_cast<f32x4*>(&vs[row * kRowF + d0 + 4 * p]) = xv[p];
+            // masked: value rows past the block are zero, as in fixed_block_kernel
+            // (an infinite last row must not meet their zero probabilities)
+            *reinterpret_cast<f32x4*>(&vs[row * kRowF + d0 + 4 * p]) =
+                MK != PISA_MASK_NONE && row >= len ? f32x4(0.0f) : xv[p];
         }
     }
     __syncthreads();
@@ -424,7 +597,9 @@ __global__ __launch_bounds__(256) void fixed_block_f32_mfma_kernel(View q, View 
         for (int r = 0; r < 4; ++r) {
             const int key = 16 * n + 4 * g + r;
             const bool dead = key >= len || (causal && key > query);
-            sacc[n][r] = dead ? -__builtin_inff() : sacc[n][r] * scale;
+            float x = sacc[n][r] * scale;
+            if constexpr (MK != PISA_MASK_NONE) x = masked_score<MK>(x, me[n], r);
+            sacc[n][r] = dead ? -__builtin_inff() : x;
             mx = fmaxf(mx, sacc[n][r]);
         }
     {
@@ -468,18 +643,6 @@ __global__ __launch_bounds__(256) void fixed_block_f32_mfma_kernel(View q, View 
         for (int j = 0; j < 4; ++j) x[j] = oacc[(f + j) % VW][(f + j) / VW];
         *reinterpret_cast<f32x4*>(dst + f) = x;
     }
-}
-
-// e^x for x <= 0 in fp32: 2^(x log2 e) on v_exp_f32, with the rounding error of
-// the product (an fma) and the low part of log2 e carried into a first-order
-// factor (its neglected square is below 1e-10 for x >= -100); -inf gives 0.
-// Four full-rate instructions and one exponential where expf's range handling
-// takes about a dozen (C1 9.43 -> 9.06 us, same error against float64).
-__device__ __forceinline__ float exp_nonpos(float x) {
-    const float hi = x * kLog2e;
-    const float lo = fmaf(x, kLog2e, -hi) + x * 1.925963e-8f;  // log2(e) - fp32(log2(e)) = 1.925963e-8
-    const float e = __builtin_amdgcn_exp2f(hi) * fmaf(lo, 0.69314718f, 1.0f);
-    return x == -__builtin_inff() ? 0.0f : e;
 }
 
 // fp32 fixed-block attention on the bf16 matrix cores (head dims 32 and 64;
@@ -682,20 +845,52 @@ __global__ __launch_bounds__(256) void fixed_block_f32x3_kernel(View q, View k, 
 
 template <typename T, int D>
 static void launch_fixed_mfma(const View& q, const View& k, const View& v, const OutView& o, int tokens, int nblocks,
-                              int bh_count, float scale, int causal, hipStream_t stream) {
-    hipLaunchKernelGGL((fixed_block_mfma_kernel<T, D>), dim3(bh_count * nblocks), dim3(64), 0, stream, q, k, v, o,
-                       tokens, nblocks, scale * kLog2e, causal);
+                              int bh_count, float scale, int causal, const MaskView& mask, hipStream_t stream) {
+    const int wide = mask.kind != PISA_MASK_NONE && mask_rows_wide(mask);
+#define PISA_FIXED_MFMA(MK)                                                                                        \
+    case MK:                                                                                                       \
+        hipLaunchKernelGGL((fixed_block_mfma_kernel<T, D, MK>), dim3(bh_count * nblocks), dim3(64), 0, stream, q, k, v, \
+                           o, tokens, nblocks, scale, causal, mask, wide);                                         \
+        break;
+    switch (mask.kind) {
+        PISA_FIXED_MFMA(PISA_MASK_NONE)
+        PISA_FIXED_MFMA(PISA_MASK_BOOL)
+        PISA_FIXED_MFMA(PISA_MASK_ADD_F32)
+        PISA_FIXED_MFMA(PISA_MASK_ADD_F16)
+        PISA_FIXED_MFMA(PISA_MASK_ADD_BF16)
+    }
+#undef PISA_FIXED_MFMA
 }
 
 template <int D>
 static void launch_fixed_f32_mfma(const View& q, const View& k, const View& v, const OutView& o, int tokens,
-                                  int nblocks, int bh_count, float scale, int causal, hipStream_t stream) {
-    if constexpr (D <= 64)
-        hipLaunchKernelGGL((fixed_block_f32x3_kernel<D>), dim3(bh_count * nblocks), dim3(256), 0, stream, q, k, v, o,
-                           tokens, nblocks, scale, causal);
-    else
-        hipLaunchKernelGGL((fixed_block_f32_mfma_kernel<D>), dim3(bh_count * nblocks), dim3(256), 0, stream, q, k, v,
-                           o, tokens, nblocks, scale, causal);
+                                  int nblocks, int bh_count, float scale, int causal, const MaskView& mask,
+                                  hipStream_t stream) {
+    if constexpr (D <= 64) {
+        if (mask.kind == PISA_MASK_NONE) {
+            hipLaunchKernelGGL((fixed_block_f32x3_kernel<D>), dim3(bh_count * nblocks), dim3(256), 0, stream, q, k, v, o,
+                               tokens, nblocks, scale, causal);
+            return;
+        }
+    }
+    const int wide = mask.kind != PISA_MASK_NONE && mask_rows_wide(mask);
+#define PISA_FIXED_F32(MK)                                                                                             \
+    case MK:                                                                                                           \
+        hipLaunchKernelGGL((fixed_block_f32_mfma_kernel<D, MK>), dim3(bh_count * nblocks), dim3(256), 0, stream, q, k, v, \
+                           o, tokens, nblocks, scale, causal, mask, wide);                                             \
+        break;
+    switch (mask.kind) {
+        case PISA_MASK_NONE:
+            if constexpr (D > 64)
+                hipLaunchKernelGGL((fixed_block_f32_mfma_kernel<D, PISA_MASK_NONE>), dim3(bh_count * nblocks), dim3(256),
+                                   0, stream, q, k, v, o, tokens, nblocks, scale, causal, mask, wide);
+            break;
+        PISA_FIXED_F32(PISA_MASK_BOOL)
+        PISA_FIXED_F32(PISA_MASK_ADD_F32)
+        PISA_FIXED_F32(PISA_MASK_ADD_F16)
+        PISA_FIXED_F32(PISA_MASK_ADD_BF16)
+    }
+#undef PISA_FIXED_F32
 }
 
 template <typename T>
@@ -712,20 +907,18 @@ int launch_fixed_t(int head_dim, const View& q, const View& k, const View& v, co
     const int out_bytes = std::is_same<T, float>::value ? 16 : 2 * head_dim / 32;
     const bool rows16 = aligned(q.data, q.sb, q.sh, q.st, 16) && aligned(k.data, k.sb, k.sh, k.st, 16) &&
                         aligned(v.data, v.sb, v.sh, v.st, 16) && aligned(o.data, o.sb, o.sh, o.st, out_bytes);
-    if constexpr (std::is_same<T, float>::value) {
-        if (mask.kind == PISA_MASK_NONE && rows16) {
-            if (head_dim == 32) launch_fixed_f32_mfma<32>(q, k, v, o, tokens, nblocks, bh_count, scale, causal, stream);
-            else if (head_dim == 64) launch_fixed_f32_mfma<64>(q, k, v, o, tokens, nblocks, bh_count, scale, causal, stream);
-            else launch_fixed_f32_mfma<128>(q, k, v, o, tokens, nblocks, bh_count, scale, causal, stream);
-            return pisa_host::check_launch("fixed_block_f32 kernel");
-        }
-    } else {
-        if (mask.kind == PISA_MASK_NONE && rows16) {  // the reference's Triton path: no mask (dispatch.py:50-79)
-            if (head_dim == 32) launch_fixed_mfma<T, 32>(q, k, v, o, tokens, nblocks, bh_count, scale, causal, stream);
-            else if (head_dim == 64) launch_fixed_mfma<T, 64>(q, k, v, o, tokens, nblocks, bh_count, scale, causal, stream);
-            else launch_fixed_mfma<T, 128>(q, k, v, o, tokens, nblocks, bh_count, scale, causal, stream);
-            return pisa_host::check_launch("fixed_block_mfma_kernel");
-        }
+    if (rows16) {
+        auto run = [&](auto dim) {
+            constexpr int D = decltype(dim)::value;
+            if constexpr (std::is_same<T, float>::value)
+                launch_fixed_f32_mfma<D>(q, k, v, o, tokens, nblocks, bh_count, scale, causal, mask, stream);
+            else
+                launch_fixed_mfma<T, D>(q, k, v, o, tokens, nblocks, bh_count, scale, causal, mask, stream);
+        };
+        if (head_dim == 32) run(std::integral_constant<int, 32>{});
+        else if (head_dim == 64) run(std::integral_constant<int, 64>{});
+        else run(std::integral_constant<int, 128>{});
+        return pisa_host::check_launch(std::is_same<T, float>::value ? "fixed_block_f32 kernel" : "fixed_block_mfma_kernel");
     }
     if (head_dim == 32)
         hipLaunchKernelGGL((fixed_block_kernel<T, 32>), grid, dim3(256), 0, stream, q, k, v, o, tokens, nblocks, scale,
