@@ -382,9 +382,9 @@ static int prepare_impl(int32_t dtype, int32_t heads, int32_t tokens, int32_t he
     int rc;
     if (head_dim != 128) {
         const int padded = pisa::padded_head_dim(head_dim);
-        if ((rc = pisa::launch_stats_means(dtype, padded, sa, bh, st, false))) return rc;
-        if ((rc = pisa::launch_kv_pack(dtype, padded, head_dim, sa.k, sa.v, sa.map, tokens, p.blocks, bh,
-                                       static_cast<char*>(w.kp), static_cast<char*>(w.vp), st)))
+        const pisa::PackMeans pm{sa.q, w.qc_route, w.kc, w.kbar_pad, w.vbar_t_pad, p.npad};
+        if ((rc = pisa::launch_kv_pack_means(dtype, padded, head_dim, sa.k, sa.v, sa.map, tokens, p.blocks, bh,
+                                             static_cast<char*>(w.kp), static_cast<char*>(w.vp), pm, st)))
             return rc;
         if (first_order) {
             // H_sum of the Triton statistics (pisa_kernel.py:80-84) from the

@@ -743,21 +743,32 @@ void attention_persistent_kernel(AttnArgs a, const int32_t* __restrict__ sel, co
 // ---- packed key and value blocks (kfrag_elem / vfrag_elem order at the
 // padded width D; dims >= d_real and rows >= kv_tokens are zero; block j
 // row r is token map(64 j + r)).  One workgroup per block: 64 rows x D of K
-// and V are read with 16-byte loads (4 rows per thread), the key fragments are
-// written straight from registers and the value block is transposed through
-// LDS.
-template <typename T, int D>
+// and V are read with 16-byte loads (kRows rows per thread, two at D = 64 so
+// that all 256 threads load), the key fragments are written straight from
+// registers and the value block is transposed through LDS.
+//
+// MEANS (generic PISA off head dim 128): the same pass reads the query rows
+// too and forms the block means q_bar, k_bar, v_bar (fp32 sums over a thread's
+// rows, then over the row groups in order, divided by the block's length), so
+// K and V are read once for both: [1,32,16384,64] 49 + 49 us as two kernels,
+// 56-58 us as one for 335 MB (63 with four rows per thread, which leaves half
+// the threads of D = 64 idle).  K and V are then read with the non-temporal
+// hint (nothing reads those rows again, and the tables written here stay in the
+// caches for the attention kernel: call 733 -> 724 us).
+template <typename T, int D, bool MEANS>
 __global__ __launch_bounds__(256) void kv_pack_kernel(View k, View v, TokenMap map, int kv_tokens, int kv_blocks,
-                                                      int d_real, char* kp, char* vp) {
+                                                      int d_real, char* kp, char* vp, PackMeans m) {
     typedef typename Elem<T>::vec8 vec8;
-    typedef T vec4 __attribute__((ext_vector_type(4)));
     constexpr int kRow = kBlock + 8;
+    constexpr int kRows = MEANS && D <= 64 ? 2 : 4;
+    typedef T vecr __attribute__((ext_vector_type(kRows)));
+    constexpr int kPieces = D / 8;            // 16-byte pieces per row
+    constexpr int kGroups = 256 / kPieces;    // row groups per pass
     __shared__ __attribute__((aligned(16))) T lds[D * kRow];
+    __shared__ float red[MEANS ? 3 : 1][MEANS ? kGroups : 1][MEANS ? D : 1];
     const int t = threadIdx.x;
     const int bh = blockIdx.x / kv_blocks;
     const int j = blockIdx.x - bh * kv_blocks;
-    constexpr int kPieces = D / 8;            // 16-byte pieces per row
-    constexpr int kRowsPerPass = 256 / kPieces;
     const int pc = t % kPieces;
     const int r0 = t / kPieces;
     const bool live_d = pc * 8 < d_real;      // d_real is a multiple of 8
@@ -765,37 +776,62 @@ __global__ __launch_bounds__(256) void kv_pack_kernel(View k, View v, TokenMap m
     T* vdst = reinterpret_cast<T*>(vp) + ((int64_t)bh * kv_blocks + j) * D * kBlock;
     const int base = map.block_base(j);          // raster token of row r: base + intra_offset(r)
     const int last = kv_tokens - 1 - j * kBlock;  // rows past the end read the last token
-    for (int r = r0 * 4; r < kBlock; r += kRowsPerPass * 4) {
-        // the 8 loads of the 4 rows go out together and unconditionally (rows
+    float sums[3][8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sums[0][e] = sums[1][e] = sums[2][e] = 0.0f;
+    for (int r = r0 * kRows; r0 < kGroups && r < kBlock; r += kGroups * kRows) {
+        // the loads of the rows go out together and unconditionally (rows
         // past kv_tokens re-read the last token, dims past d_real the first
         // piece; both are zeroed at use), so no load waits behind another
-        vec8 kx[4], x[4];
-        bool live[4];
+        vec8 qx[MEANS ? kRows : 1], kx[kRows], x[kRows];
+        bool live[kRows];
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
+        for (int rr = 0; rr < kRows; ++rr) {
             const int key = j * kBlock + r + rr;
             live[rr] = key < kv_tokens && live_d;
             const int tok = base + map.intra_offset(min(r + rr, last));
             const int dc = live_d ? pc * 8 : 0;
-            kx[rr] = load8<vec8>(k.data + (k.row(bh, tok) + dc) * sizeof(T));
-            x[rr] = load8<vec8>(v.data + (v.row(bh, tok) + dc) * sizeof(T));
+            if constexpr (MEANS) qx[rr] = load8<vec8>(m.q.data + (m.q.row(bh, tok) + dc) * sizeof(T));
+            const char* krow = k.data + (k.row(bh, tok) + dc) * sizeof(T);
+            const char* vrow = v.data + (v.row(bh, tok) + dc) * sizeof(T);
+            kx[rr] = MEANS ? load8_nt<vec8>(krow) : load8<vec8>(krow);
+            x[rr] = MEANS ? load8_nt<vec8>(vrow) : load8<vec8>(vrow);
         }
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
+        for (int rr = 0; rr < kRows; ++rr) {
             if (!live[rr]) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
+                    if constexpr (MEANS) qx[rr][e] = T(0.0f);
                     kx[rr][e] = T(0.0f);
                     x[rr][e] = T(0.0f);
                 }
             }
             store8(kdst + kfrag_elem(r + rr, pc * 8, D), kx[rr]);
+            if constexpr (MEANS) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    sums[0][e] += to_f32(qx[rr][e]);
+                    sums[1][e] += to_f32(kx[rr][e]);
+                    sums[2][e] += to_f32(x[rr][e]);
+                }
+            }
         }
-        const int p = swap23(r);
+        const int p = swap23(r);  // rows r .. r + kRows - 1 stay consecutive
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            vec4 w = {x[0][e], x[1][e], x[2][e], x[3][e]};
-            *reinterpret_cast<vec4*>(&lds[(pc * 8 + e) * kRow + p]) = w;
+            vecr w;
+#pragma unroll
+            for (int rr = 0; rr < kRows; ++rr) w[rr] = x[rr][e];
+            *reinterpret_cast<vecr*>(&lds[(pc * 8 + e) * kRow + p]) = w;
+        }
+    }
+    if constexpr (MEANS) {
+        if (r0 < kGroups) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) red[i][r0][pc * 8 + e] = sums[i][e];
         }
     }
     __syncthreads();
@@ -806,6 +842,32 @@ __global__ __launch_bounds__(256) void kv_pack_kernel(View k, View v, TokenMap m
         const int row = (f >> 2) * 32 + (L & 31);
         const int pos = (f & 3) * 16 + (L >> 5) * 8;
         store8(vdst + id * 8, *reinterpret_cast<const vec8*>(&lds[row * kRow + pos]));
+    }
+    if constexpr (MEANS) {
+        const float len = static_cast<float>(min(kBlock, kv_tokens - j * kBlock));
+        const int64_t head_base = (int64_t)bh * m.npad * D;
+        const int64_t chunk_base = head_base + (int64_t)(j & ~63) * D;  // packed 64-centroid chunk
+        for (int id = t; id < 3 * D; id += 256) {
+            const int which = id / D;
+            const int d = id - which * D;
+            float s = 0.0f;
+#pragma unroll
+            for (int g = 0; g < kGroups; ++g) s += red[which][g][d];
+            s /= len;  // dims past d_real are zero
+            const int64_t o = ((int64_t)bh * kv_blocks + j) * d_real + d;
+            T* pack = which == 1 ? static_cast<T*>(m.kbar_pad) : static_cast<T*>(m.vbar_t_pad);
+            auto elem = [&](int c) { return which == 1 ? kfrag_elem(c, d, D) : vfrag_elem(c, d); };
+            if (which == 0) {
+                if (d < d_real) m.q_mean[o] = s;
+                continue;
+            }
+            if (which == 1 && d < d_real) m.k_mean[o] = s;
+            pack[chunk_base + elem(j & 63)] = from_f32<T>(s);
+            if (j == kv_blocks - 1)
+                // centroids past the last block: masked to -inf in the tail, zero here
+                // so that 0 * value stays finite in the PV product
+                for (int c = kv_blocks; c < m.npad; ++c) pack[head_base + (int64_t)(c & ~63) * D + elem(c & 63)] = T(0.0f);
+        }
     }
 }
 
@@ -890,14 +952,14 @@ int launch_attention(int dtype, int padded, bool sparse, bool tail, const AttnAr
     return launch_attention_dt<f16_t>(padded, sparse, tail, a, bh_count, stream);
 }
 
-template <typename T>
+template <typename T, bool MEANS>
 int launch_kv_pack_t(int padded, int head_dim, const View& k, const View& v, TokenMap map, int kv_tokens,
-                     int kv_blocks, int bh_count, char* kp, char* vp, hipStream_t stream) {
+                     int kv_blocks, int bh_count, char* kp, char* vp, const PackMeans& m, hipStream_t stream) {
     const dim3 grid(bh_count * kv_blocks);
-#define PISA_KV_PACK(DP)                                                                                     \
-    case DP:                                                                                                 \
-        hipLaunchKernelGGL((kv_pack_kernel<T, DP>), grid, dim3(256), 0, stream, k, v, map, kv_tokens, kv_blocks, \
-                           head_dim, kp, vp);                                                                \
+#define PISA_KV_PACK(DP)                                                                                         \
+    case DP:                                                                                                     \
+        hipLaunchKernelGGL((kv_pack_kernel<T, DP, MEANS>), grid, dim3(256), 0, stream, k, v, map, kv_tokens, kv_blocks, \
+                           head_dim, kp, vp, m);                                                                 \
         break;
     switch (padded) {
         PISA_KV_PACK(64)
@@ -914,9 +976,20 @@ int launch_kv_pack_t(int padded, int head_dim, const View& k, const View& v, Tok
 
 int launch_kv_pack(int dtype, int padded, int head_dim, const View& k, const View& v, TokenMap map, int kv_tokens,
                    int kv_blocks, int bh_count, char* kp, char* vp, hipStream_t stream) {
+    const PackMeans none{};
     if (dtype == PISA_DTYPE_BF16)
-        return launch_kv_pack_t<bf16_t>(padded, head_dim, k, v, map, kv_tokens, kv_blocks, bh_count, kp, vp, stream);
-    return launch_kv_pack_t<f16_t>(padded, head_dim, k, v, map, kv_tokens, kv_blocks, bh_count, kp, vp, stream);
+        return launch_kv_pack_t<bf16_t, false>(padded, head_dim, k, v, map, kv_tokens, kv_blocks, bh_count, kp, vp, none,
+                                               stream);
+    return launch_kv_pack_t<f16_t, false>(padded, head_dim, k, v, map, kv_tokens, kv_blocks, bh_count, kp, vp, none,
+                                          stream);
+}
+
+int launch_kv_pack_means(int dtype, int padded, int head_dim, const View& k, const View& v, TokenMap map, int kv_tokens,
+                         int kv_blocks, int bh_count, char* kp, char* vp, const PackMeans& m, hipStream_t stream) {
+    if (dtype == PISA_DTYPE_BF16)
+        return launch_kv_pack_t<bf16_t, true>(padded, head_dim, k, v, map, kv_tokens, kv_blocks, bh_count, kp, vp, m,
+                                              stream);
+    return launch_kv_pack_t<f16_t, true>(padded, head_dim, k, v, map, kv_tokens, kv_blocks, bh_count, kp, vp, m, stream);
 }
 #endif  // PISA_ATTENTION_DENSE
 

@@ -207,6 +207,19 @@ int launch_attention_d64(int dtype, bool sparse, const AttnArgs& a, int bh_count
 // block j row r is token map(64 j + r).
 int launch_kv_pack(int dtype, int padded, int head_dim, const View& k, const View& v, TokenMap map, int kv_tokens,
                    int kv_blocks, int bh_count, char* kp, char* vp, hipStream_t stream);
+// The same with the block means of q, k and v from the same pass (generic PISA
+// off head dim 128): fp32 means [BH][N][head_dim] of q and k, and the packed
+// centroid chunks at the padded width (zero past the last block).
+struct PackMeans {
+    View q;
+    float* q_mean;
+    float* k_mean;
+    void* kbar_pad;
+    void* vbar_t_pad;
+    int npad;
+};
+int launch_kv_pack_means(int dtype, int padded, int head_dim, const View& k, const View& v, TokenMap map, int kv_tokens,
+                         int kv_blocks, int bh_count, char* kp, char* vp, const PackMeans& m, hipStream_t stream);
 // Fixed-block attention mask, broadcast to [B][heads][T][T] by element strides.
 struct MaskView {
     const char* data;

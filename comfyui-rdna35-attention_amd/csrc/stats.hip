@@ -364,9 +364,8 @@ __device__ __forceinline__ vec8 load_piece(const char* row, int d0, int head_dim
 // in fp32; an LDS pass adds the R row groups in order.  Means are sum / len
 // for the generic statistics (generic_pisa.py:128-132, pisa_kernel.py:72-77)
 // and sum * fp32(1/len) for the HYD statistics (pisa_kernels.cu:207-209).
-// Writes the [BH][N][D] means and, for the attention kernel, the packed
-// centroid chunks at the padded width DP (zero in dims >= D and for the
-// centroids past the last block).
+// Writes the [BH][N][D] means (the generic forward takes its own from
+// kv_pack_kernel, which reads the rows anyway).
 template <typename T, int DP, bool HYD>
 __global__ __launch_bounds__(256) void stats_means_kernel(StatsArgs a) {
     typedef typename Elem<T>::vec8 vec8;
@@ -444,23 +443,6 @@ __global__ __launch_bounds__(256) void stats_means_kernel(StatsArgs a) {
             static_cast<float*>(a.vm_out)[o] = a.vm_sums ? v_sum : mv;
         } else {
             static_cast<T*>(a.vm_out)[o] = from_f32<T>(mv);
-        }
-        if (a.qc_route) a.qc_route[o] = mq;
-    }
-    if (!a.kbar_pad) return;  // the standalone statistics entry point wants no packed centroids
-    const int64_t head_base = (int64_t)bh * a.npad * DP;
-    T* kbar = static_cast<T*>(a.kbar_pad);
-    T* vbar = static_cast<T*>(a.vbar_t_pad);
-    const int64_t chunk_base = head_base + (int64_t)(b & ~63) * DP;
-    kbar[chunk_base + kfrag_elem(b & 63, d, DP)] = live ? from_f32<T>(mk) : T(0.0f);
-    vbar[chunk_base + vfrag_elem(b & 63, d)] = live ? from_f32<T>(mv) : T(0.0f);
-    if (b == a.blocks - 1) {
-        // centroids past the last block: masked to -inf in the tail, zero here
-        // so that 0 * value stays finite in the PV product
-        for (int j = a.blocks; j < a.npad; ++j) {
-            const int64_t base = head_base + (int64_t)(j & ~63) * DP;
-            kbar[base + kfrag_elem(j & 63, d, DP)] = T(0.0f);
-            vbar[base + vfrag_elem(j & 63, d)] = T(0.0f);
         }
     }
 }
