@@ -176,6 +176,7 @@ def _launch_dense(q4, k4, v4, out4, scale):
         )
 
 
+_FIXED_BLOCK_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 _MASK_KINDS = {torch.bool: _lib.MASK_BOOL, torch.float32: _lib.MASK_ADD_F32, torch.float16: _lib.MASK_ADD_F16,
                torch.bfloat16: _lib.MASK_ADD_BF16}
 
@@ -247,7 +248,10 @@ def _eager(*tensors) -> bool:
     """True outside a compiler trace when every tensor is a plain torch.Tensor (not fake/functional)."""
     if torch.compiler.is_compiling():
         return False
-    return all(type(t) is torch.Tensor for t in tensors if t is not None)
+    for t in tensors:
+        if t is not None and type(t) is not torch.Tensor:
+            return False
+    return True
 
 
 def _forward_kernel(q, k, v, exact_blocks: int, scale: float, sink_block: int) -> torch.Tensor:
@@ -545,8 +549,13 @@ def fixed_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sca
     (broadcast dims as 0 strides): bool keeps a score where True, a float mask
     is added to the scaled scores (reference.py:186-195).
     """
-    _check_inputs("fixed-block attention", q, k, v, dtypes=(torch.bfloat16, torch.float16, torch.float32),
-                  same_tokens=True)
+    _check_fixed_block(q, k, v, mask)
+    fn = _fixed_block_kernel if _eager(q, k, v, mask) else _fixed_block_op
+    return fn(q, k, v, float(scale), bool(causal), mask)
+
+
+def _check_fixed_block(q, k, v, mask) -> None:
+    _check_inputs("fixed-block attention", q, k, v, dtypes=_FIXED_BLOCK_DTYPES, same_tokens=True)
     if mask is not None:
         batch, heads, tokens, _ = q.shape
         if not isinstance(mask, torch.Tensor) or mask.ndim != 4 or mask.device != q.device:
@@ -554,8 +563,12 @@ def fixed_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sca
         if tuple(mask.shape[2:]) != (tokens, tokens) or mask.shape[0] * mask.shape[1] != batch * heads:
             raise ValueError(f"fixed-block mask must be [B',H',{tokens},{tokens}] with B'*H' = {batch * heads}, "
                              f"got {tuple(mask.shape)}")
-    fn = _fixed_block_kernel if _eager(q, k, v, mask) else _fixed_block_op
-    return fn(q, k, v, float(scale), bool(causal), mask)
+
+
+def _fixed_block_into(q, k, v, out, scale: float, causal: bool, mask) -> None:
+    """fixed_block_attention of plain tensors into `out`, a [B,H,T,D] view of any aligned layout."""
+    _check_fixed_block(q, k, v, mask)
+    _launch_fixed_block(q, k, v, out, float(scale), bool(causal), mask)
 
 
 def route_topk(q_centroids: torch.Tensor, k_centroids: torch.Tensor, h_norm: torch.Tensor | None,

@@ -195,10 +195,13 @@ def stream_of(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+_NO_GUARD = contextlib.nullcontext()  # stateless
+
+
 def on_device(device: torch.device):
     """Device guard around a launch; a no-op when `device` is already the current device."""
     if device.index is None or device.index == torch.cuda.current_device():
-        return contextlib.nullcontext()
+        return _NO_GUARD
     return torch.cuda.device(device)
 
 

@@ -1,0 +1,81 @@
+"""Fixed-block dispatch on tensors the kernels read in place, against the same call on contiguous copies.
+
+The copies take the route every call took before (normalised to contiguous [BH,T,D]); both ways run one kernel on the
+same rows, so the results are equal bit for bit, shape and strides included.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from rdna35_block_attention import dispatch, fixed_block_attention
+
+B, H, T, D = 2, 3, 150, 64
+
+
+def _bhtd(form, gen, dtype):
+    def one():
+        if form == "contiguous":
+            return torch.randn((B, H, T, D), generator=gen).to(dtype)
+        if form == "transposed":          # [B,T,H,D] storage
+            return torch.randn((B, T, H, D), generator=gen).to(dtype).transpose(1, 2)
+        if form == "sliced_heads":
+            return torch.randn((B, 2 * H, T, D), generator=gen).to(dtype)[:, ::2]
+        if form == "odd_rows":            # rows of D + 1 elements: not 16-byte aligned
+            return torch.randn((B, H, T, D + 1), generator=gen).to(dtype)[..., :D]
+        return torch.randn((B, H, D, T), generator=gen).to(dtype).transpose(2, 3)  # "strided_dims"
+    return one(), one(), one()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("form", ["contiguous", "transposed", "sliced_heads", "odd_rows", "strided_dims"])
+@pytest.mark.parametrize("mask_kind", [None, "2d", "4d"])
+def test_bhtd_views_match_contiguous_copies(monkeypatch, dtype, form, mask_kind):
+    gen = torch.Generator().manual_seed(11)
+    q, k, v = (t.cuda() for t in _bhtd(form, gen, dtype))
+    q, k, v = (t if form == "contiguous" else _like(t, form) for t in (q, k, v))
+    mask = {None: None, "2d": torch.rand((T, T), generator=gen) < 0.8,
+            "4d": torch.randn((B, 1, T, T), generator=gen)}[mask_kind]
+    mask = None if mask is None else mask.cuda()
+    out = fixed_block_attention(q, k, v, layout="bhtd", causal=True, mask=mask)
+    monkeypatch.setattr(dispatch, "_in_place_views", lambda *args: None)
+    before = fixed_block_attention(q, k, v, layout="bhtd", causal=True, mask=mask)
+    assert out.shape == before.shape and out.stride() == before.stride()
+    assert torch.equal(torch.nan_to_num(out, nan=7.0), torch.nan_to_num(before, nan=7.0))
+
+
+def _like(t, form):
+    """t on the GPU with the strides its form names (a device copy of a view is contiguous)."""
+    if form == "transposed":
+        return t.transpose(1, 2).contiguous().transpose(1, 2)
+    if form == "sliced_heads":
+        return torch.stack((t, t), dim=2).flatten(1, 2)[:, ::2]
+    if form == "odd_rows":
+        return torch.nn.functional.pad(t, (0, 1))[..., :D]
+    return t.transpose(2, 3).contiguous().transpose(2, 3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fused", [False, True])
+def test_bthd_layout_matches_contiguous_copies(monkeypatch, fused):
+    """[B,T,H*D] calls, also as a third of one fused projection, store [B,T,H*D] directly."""
+    gen = torch.Generator().manual_seed(12)
+    x = torch.randn((B, T, 3 * H * D), generator=gen).to(torch.float16).cuda()
+    q, k, v = x.chunk(3, dim=2)
+    if not fused:
+        q, k, v = (t.contiguous() for t in (q, k, v))
+    out, info = fixed_block_attention(q, k, v, layout="bthd", heads=H, return_diagnostics=True)
+    monkeypatch.setattr(dispatch, "_in_place_views", lambda *args: None)
+    before, info_before = fixed_block_attention(q, k, v, layout="bthd", heads=H, return_diagnostics=True)
+    assert out.stride() == before.stride() and torch.equal(out, before) and info == info_before
+
+
+def test_rows_readable_needs_unit_stride_and_aligned_rows():
+    x = torch.zeros((B, H, T, D), dtype=torch.bfloat16)
+    assert dispatch._rows_readable(x) and dispatch._rows_readable(x.transpose(0, 1))
+    assert not dispatch._rows_readable(x.transpose(2, 3))
+    assert not dispatch._rows_readable(torch.zeros((B, H, T, D + 4), dtype=torch.bfloat16)[..., :D])
+    assert dispatch._rows_readable(torch.zeros((B, H, T, D + 4), dtype=torch.float32)[..., :D])
+    assert not dispatch._rows_readable(torch.zeros(B * H * T * D + 1, dtype=torch.bfloat16)[1:].view(B, H, T, D))
+    assert dispatch._in_place_views(x, x, x, "bhtd", None) is None  # CPU tensors take the eager route
