@@ -34,9 +34,18 @@ constexpr int kRawFlags = 0x00020000;  // untyped 32-bit buffer data format
 // result is reproducible): per column the running maxima, then the parts of O
 // scaled to the common maximum and summed by output units.  Every key and value
 // byte is still loaded once per query block.  launch_t chooses W.
-template <typename T, bool SPARSE, bool TAIL, int W>
+//
+// DIRECT (small dense calls): K and V are read from the caller's rows instead of
+// the packed tables, so no packing launch runs before.  The key operand is 16
+// bytes of one row per lane; of the values a lane reads two consecutive dims of
+// every key row it contracts (as in fixed_block_mfma_kernel), so output tile md
+// holds dims 2i + md of accumulator row i.  Each chunk costs more loads (20
+// instead of 8 per half, of 32 separate rows each): dense_rows_d64 says when
+// that is the better trade.
+template <typename T, bool SPARSE, bool TAIL, int W, bool DIRECT>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uint32_t* __restrict__ selmask) {
+    static_assert(!DIRECT || (!SPARSE && !TAIL), "rows are read in place by the dense kernel only");
     typedef typename Elem<T>::vec8 vec8;
     const int lane = threadIdx.x & 63;
     const int wave = W > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
@@ -107,6 +116,18 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
         (void*)(TAIL ? a.vbar_t + (int64_t)bh * a.npad * kD * 2 : a.vp), (short)0, cen_bytes, kRawFlags);
     const int lane_off = lane * 16;
 
+    // DIRECT: the rows of this head; rows past the last read as zero
+    const int k_row = DIRECT ? (int)a.k.st * 2 : 0, v_row = DIRECT ? (int)a.v.st * 2 : 0;  // bytes
+    const __amdgpu_buffer_rsrc_t kr_rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(DIRECT ? a.k.data + a.k.row(bh, 0) * 2 : a.kp), (short)0,
+        DIRECT ? (a.kv_tokens - 1) * k_row + a.head_dim * 2 : 0, kRawFlags);
+    const __amdgpu_buffer_rsrc_t vr_rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(DIRECT ? a.v.data + a.v.row(bh, 0) * 2 : a.vp), (short)0,
+        DIRECT ? (a.kv_tokens - 1) * v_row + a.head_dim * 2 : 0, kRawFlags);
+    const int k_lane = col * k_row + half * 16;
+    const int v_lane = 4 * half * v_row + col * 4;
+    const bool all_dims = a.head_dim >= kD;
+
     auto is_tail = [&](int x) { return TAIL && min(x, n_chunks - 1) >= n_exact; };
     auto table_row = [&](int x) -> int {  // block id, or centroid chunk id; past the list, its last chunk again
         x = min(x, n_chunks - 1);
@@ -120,12 +141,31 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
     };
 
     vec8 kf[KT];     // key fragments of the half chunk scored next
-    vec8 vf[MD][2];  // value fragments of the half chunk multiplied next
+    vec8 vf[DIRECT ? 1 : MD][2];  // value fragments of the half chunk multiplied next
+    uint32_t vr[DIRECT ? 2 : 1][8];  // DIRECT: dims 2col, 2col + 1 of its keys 16ss + 8(e/4) + 4half + e%4
     auto load_k = [&](bool tail, int row, int mt) {
+        if constexpr (DIRECT) {
+            const int soff = __builtin_amdgcn_readfirstlane((row * kBlock + mt * 32) * k_row);
+#pragma unroll
+            for (int t = 0; t < KT; ++t)
+                kf[t] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(kr_rs, k_lane + t * 32, soff, 0));
+            return;
+        }
 #pragma unroll
         for (int t = 0; t < KT; ++t) kf[t] = ld_frag(tail ? kc_rs : kp_rs, row * kBlockBytes, mt * KT + t);
     };
     auto load_v = [&](bool tail, int row, int mt) {
+        if constexpr (DIRECT) {
+#pragma unroll
+            for (int ss = 0; ss < 2; ++ss)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int key = row * kBlock + mt * 32 + 16 * ss + 8 * (e >> 2) + (e & 3);
+                    vr[ss][e] = __builtin_amdgcn_raw_buffer_load_b32(vr_rs, v_lane,
+                                                                     __builtin_amdgcn_readfirstlane(key * v_row), 0);
+                }
+            return;
+        }
 #pragma unroll
         for (int md = 0; md < MD; ++md)
 #pragma unroll
@@ -165,6 +205,13 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int v = 0; v < 16; ++v) s[nt][v] = 0.0f;
+        if constexpr (DIRECT) {
+            if (!all_dims) {  // what lies past a narrower row must not meet the zero query dims
+#pragma unroll
+                for (int t = 0; t < KT; ++t)
+                    if (t * 16 + half * 8 >= a.head_dim) kf[t] = vec8(T(0.0f));
+            }
+        }
 #pragma unroll
         for (int t = 0; t < KT; ++t)
 #pragma unroll
@@ -179,9 +226,20 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
 #pragma unroll
         for (int ss = 0; ss < 2; ++ss)
 #pragma unroll
-            for (int md = 0; md < MD; ++md)
+            for (int md = 0; md < MD; ++md) {
+                vec8 f;
+                if constexpr (DIRECT) {  // the 16-bit halves md of the 8 keys' words
+                    u32x4 w;
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt) o[md][nt] = mfma32(vf[md][ss], pf[nt][ss], o[md][nt]);
+                    for (int j = 0; j < 4; ++j)
+                        w[j] = __builtin_amdgcn_perm(vr[ss][2 * j + 1], vr[ss][2 * j], md ? 0x07060302u : 0x05040100u);
+                    f = __builtin_bit_cast(vec8, w);
+                } else {
+                    f = vf[md][ss];
+                }
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) o[md][nt] = mfma32(f, pf[nt][ss], o[md][nt]);
+            }
     };
     // column maxima and running-max update of half mt of a chunk; `plain`: an
     // exact full block, else a short last key block is masked first
@@ -299,10 +357,28 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
     for (int u = 0; u < kUnits / W; ++u) {
         // W = 1: tile and pair are constants and the accumulators stay in registers
         const int unit = wave * (kUnits / W) + u;
-        const int p = unit & 1, nt = (unit >> 1) & 1, md = unit >> 2;
+        // DIRECT: unit = accumulator group g of query tile nt over both tiles md
+        // (dims 16g + 8half .. +7 of a lane's query)
+        const int p = unit & 1, nt = DIRECT ? unit >> 2 : (unit >> 1) & 1, md = DIRECT ? 0 : unit >> 2;
         const bool second = nt != 0;
         float x[8];
-        if constexpr (W > 1) {
+        if constexpr (DIRECT) {
+            const int g = unit & 3;
+#pragma unroll
+            for (int d = 0; d < MD; ++d) {
+                f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (W > 1) {
+#pragma unroll
+                    for (int w = 0; w < W; ++w)
+                        sum += *reinterpret_cast<const f32x4*>(&parts[((((w * MD + d) * NT + nt) * 4 + g) * 64 + lane) * 4]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sum[e] = o[d][u >> 2][4 * (u & 3) + e];
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[MD * e + d] = sum[e];
+            }
+        } else if constexpr (W > 1) {
 #pragma unroll
             for (int g = 0; g < 2; ++g) {
                 f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -343,6 +419,17 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
 #pragma unroll
             for (int e = 0; e < 4; ++e) out[e] = from_f32<T>(x[4 * g + e]);
             w4[g] = __builtin_bit_cast(u32x2, out);
+        }
+        if constexpr (DIRECT) {
+            const int d = 16 * (unit & 3) + 8 * half;
+            if (d >= a.head_dim) continue;
+            if (st16) {
+                *reinterpret_cast<u32x4*>(dst + d * sizeof(T)) = u32x4{w4[0][0], w4[0][1], w4[1][0], w4[1][1]};
+            } else {
+                *reinterpret_cast<u32x2*>(dst + d * sizeof(T)) = w4[0];
+                *reinterpret_cast<u32x2*>(dst + (d + 4) * sizeof(T)) = w4[1];
+            }
+            continue;
         }
         if (st16) {
             // one lane-half swap per dword leaves lanes 0-31 with dims 8(2p) .. +7 and
@@ -397,14 +484,14 @@ int waves_per_block(int64_t blocks, int n_chunks) {
     return best;
 }
 
-template <typename T, bool SPARSE, bool TAIL>
+template <typename T, bool SPARSE, bool TAIL, bool DIRECT>
 int launch_t(const AttnArgs& a, int bh_count, hipStream_t stream) {
     const int blocks = bh_count * a.q_blocks;
     const int n_chunks = (SPARSE ? a.exact : a.kv_blocks) + (TAIL ? a.npad / kBlock : 0);
     const int w = waves_per_block(blocks, n_chunks);
-#define PISA_D64(W)                                                                                              \
-    hipLaunchKernelGGL((attention_d64_kernel<T, SPARSE, TAIL, W>), dim3(blocks), dim3(64 * W), 0, stream, a, a.idx, \
-                       a.selmask)
+#define PISA_D64(W)                                                                                            \
+    hipLaunchKernelGGL((attention_d64_kernel<T, SPARSE, TAIL, W, DIRECT>), dim3(blocks), dim3(64 * W), 0, stream, a, \
+                       a.idx, a.selmask)
     if (w == 1) PISA_D64(1);
     else if (w == 2) PISA_D64(2);
     else if (w == 4) PISA_D64(4);
@@ -417,10 +504,30 @@ int launch_t(const AttnArgs& a, int bh_count, hipStream_t stream) {
 
 int launch_attention_d64(int dtype, bool sparse, const AttnArgs& a, int bh_count, hipStream_t stream) {
     if (dtype == PISA_DTYPE_BF16)
-        return sparse ? launch_t<bf16_t, true, true>(a, bh_count, stream)
-                      : launch_t<bf16_t, false, false>(a, bh_count, stream);
-    return sparse ? launch_t<f16_t, true, true>(a, bh_count, stream)
-                  : launch_t<f16_t, false, false>(a, bh_count, stream);
+        return sparse ? launch_t<bf16_t, true, true, false>(a, bh_count, stream)
+                      : launch_t<bf16_t, false, false, false>(a, bh_count, stream);
+    return sparse ? launch_t<f16_t, true, true, false>(a, bh_count, stream)
+                  : launch_t<f16_t, false, false, false>(a, bh_count, stream);
+}
+
+// Reading rows in place saves the packing launch (about 4.5 us and 6.7 ns a key
+// block: 3.5 us for [1,8,1000,64], 11.3 us for [2,10,4096,64]) and costs 0.2 to
+// 0.4 ns for every chunk that a query block walks, so the line lies where
+// 0.35 ns x (query blocks x chunks) reaches it.  Packed -> in place, one MI355X:
+// [1,8,1000,64] 20.0 -> 16.9 us (host time of the launch included), [2,20,1024,64]
+// 30.1 -> 25.2, [2,10,2048,64] 45.9 -> 45.1, 64 keys of 4096 tokens in 32 heads
+// 19.3 -> 16.3; on the other side [2,20,2048,64] 62.2 -> 62.4, [1,8,4096,64]
+// 65.1 -> 69.5, [2,24,9216,64] x 512 keys 80.5 -> 89.3, [2,16,4096,64] 155 -> 164.
+// The rows of a head are addressed with 32-bit byte offsets.
+bool dense_rows_d64(const AttnArgs& a, int bh_count) {
+    auto addressable = [&](const View& x) { return x.st > 0 && x.st <= INT32_MAX / 2 / a.kv_tokens - 1; };
+    const int64_t chunks = (int64_t)bh_count * a.q_blocks * a.kv_blocks;
+    return chunks < 13000 + 19 * (int64_t)bh_count * a.kv_blocks && addressable(a.k) && addressable(a.v);
+}
+
+int launch_attention_d64_rows(int dtype, const AttnArgs& a, int bh_count, hipStream_t stream) {
+    return dtype == PISA_DTYPE_BF16 ? launch_t<bf16_t, false, false, true>(a, bh_count, stream)
+                                    : launch_t<f16_t, false, false, true>(a, bh_count, stream);
 }
 
 }  // namespace pisa

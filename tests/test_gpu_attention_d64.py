@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -40,15 +41,40 @@ def native():
     (20, 1600, 512, 64),    # 500 blocks of 8 chunks: two waves
     (64, 1024, 130, 64),    # 1024 blocks: one wave
     (2, 64, 449, 8),        # eight waves on eight chunks, one each
+    # the shapes above read K and V in place, these from packed tables
+    (1, 7990, 8000, 64),    # 125 blocks of 125 chunks: eight waves
+    (2, 6400, 6400, 40),    # 200 blocks: four waves
+    (5, 6400, 2500, 64),    # 500 blocks of 40 chunks: two waves
+    (16, 4096, 1279, 64),   # 1024 blocks of 20 chunks: one wave
 ])
 def test_dense_splits_match_oracle(native, dtype, heads, q_tokens, kv_tokens, head_dim):
     gen = torch.Generator().manual_seed(heads * 7 + q_tokens + kv_tokens)
     q = torch.randn((1, heads, q_tokens, head_dim), generator=gen).to(dtype)
     k, v = (torch.randn((1, heads, kv_tokens, head_dim), generator=gen).to(dtype) for _ in range(2))
     out = native.dense_attention(q.cuda(), k.cuda(), v.cuda(), 1 / math.sqrt(head_dim))
-    expected = oatt.dense_attention(np32(q), np32(k), np32(v))
+    rows = slice(None, None, 1 + q_tokens // 200)  # of a long call, some rows of every block
+    expected = oatt.dense_attention(np32(q[:, :, rows]), np32(k), np32(v))
     atol = 4 * UNIT[dtype] * float(v.float().abs().max())
-    assert_close(np32(out), expected, atol, 0.0, f"dense {heads}x{q_tokens}x{kv_tokens} D={head_dim}")
+    assert_close(np32(out[:, :, rows]), expected, atol, 0.0, f"dense {heads}x{q_tokens}x{kv_tokens} D={head_dim}")
+
+
+@pytest.mark.parametrize("head_dim,kv_tokens", [(64, 130), (40, 257), (8, 64)])
+def test_rows_read_in_place_stay_inside_their_heads(native, head_dim, kv_tokens):
+    """Views into one fused [B,T,3,H,D+8] tensor whose other elements are NaN: nothing past a row or past the last
+    token reaches the result, an infinite value in the last row stays one column's, and stores end with the row."""
+    gen = torch.Generator().manual_seed(head_dim)
+    fused = torch.full((2, kv_tokens, 3, 3, head_dim + 8), float("nan"), dtype=torch.bfloat16)
+    fused[..., :head_dim] = torch.randn((2, kv_tokens, 3, 3, head_dim), generator=gen).to(torch.bfloat16)
+    fused[0, -1, 2, 1, 3] = float("inf")
+    fused = fused.cuda()
+    q, k, v = (fused[:, :, i, :, :head_dim].transpose(1, 2) for i in range(3))
+    out = torch.full((2, 3, kv_tokens, head_dim + 4), 3.0, dtype=torch.bfloat16, device="cuda")  # 8-byte aligned rows
+    native._launch_dense(q, k, v, out[..., :head_dim], head_dim ** -0.5)
+    expected = oatt.dense_attention(np32(q), np32(k), np32(v))
+    assert np.isinf(expected[0, 1, :, 3]).all() and np.isfinite(np.delete(expected, 3, axis=3)).all()
+    atol = 4 * UNIT[torch.bfloat16] * 5.0  # |v| < 5
+    assert_close(np32(out[..., :head_dim]), expected, atol, 0.0, "in place")
+    assert bool((out[..., head_dim:] == 3.0).all())
 
 
 def test_dense_split_parts_of_very_different_scale(native):
