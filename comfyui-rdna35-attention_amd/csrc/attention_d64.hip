@@ -116,7 +116,9 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
         (void*)(TAIL ? a.vbar_t + (int64_t)bh * a.npad * kD * 2 : a.vp), (short)0, cen_bytes, kRawFlags);
     const int lane_off = lane * 16;
 
-    // DIRECT: the rows of this head; rows past the last read as zero
+    // DIRECT: the rows of this head.  The whole byte offset of a load is its
+    // vector offset, which the hardware checks against the size, so what lies
+    // past the last row (or past its last dim) reads as zero.
     const int k_row = DIRECT ? (int)a.k.st * 2 : 0, v_row = DIRECT ? (int)a.v.st * 2 : 0;  // bytes
     const __amdgpu_buffer_rsrc_t kr_rs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(DIRECT ? a.k.data + a.k.row(bh, 0) * 2 : a.kp), (short)0,
@@ -124,8 +126,6 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
     const __amdgpu_buffer_rsrc_t vr_rs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(DIRECT ? a.v.data + a.v.row(bh, 0) * 2 : a.vp), (short)0,
         DIRECT ? (a.kv_tokens - 1) * v_row + a.head_dim * 2 : 0, kRawFlags);
-    const int k_lane = col * k_row + half * 16;
-    const int v_lane = 4 * half * v_row + col * 4;
     const bool all_dims = a.head_dim >= kD;
 
     auto is_tail = [&](int x) { return TAIL && min(x, n_chunks - 1) >= n_exact; };
@@ -145,10 +145,10 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
     uint32_t vr[DIRECT ? 2 : 1][8];  // DIRECT: dims 2col, 2col + 1 of its keys 16ss + 8(e/4) + 4half + e%4
     auto load_k = [&](bool tail, int row, int mt) {
         if constexpr (DIRECT) {
-            const int soff = __builtin_amdgcn_readfirstlane((row * kBlock + mt * 32) * k_row);
+            const int off = (row * kBlock + mt * 32 + col) * k_row + half * 16;
 #pragma unroll
             for (int t = 0; t < KT; ++t)
-                kf[t] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(kr_rs, k_lane + t * 32, soff, 0));
+                kf[t] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(kr_rs, off + t * 32, 0, 0));
             return;
         }
 #pragma unroll
@@ -156,14 +156,13 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
     };
     auto load_v = [&](bool tail, int row, int mt) {
         if constexpr (DIRECT) {
+            const int off = (row * kBlock + mt * 32 + 4 * half) * v_row + col * 4;
 #pragma unroll
             for (int ss = 0; ss < 2; ++ss)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int key = row * kBlock + mt * 32 + 16 * ss + 8 * (e >> 2) + (e & 3);
-                    vr[ss][e] = __builtin_amdgcn_raw_buffer_load_b32(vr_rs, v_lane,
-                                                                     __builtin_amdgcn_readfirstlane(key * v_row), 0);
-                }
+                for (int e = 0; e < 8; ++e)
+                    vr[ss][e] = __builtin_amdgcn_raw_buffer_load_b32(
+                        vr_rs, off + (16 * ss + 8 * (e >> 2) + (e & 3)) * v_row, 0, 0);
             return;
         }
 #pragma unroll
@@ -518,9 +517,10 @@ int launch_attention_d64(int dtype, bool sparse, const AttnArgs& a, int bh_count
 // 30.1 -> 25.2, [2,10,2048,64] 45.9 -> 45.1, 64 keys of 4096 tokens in 32 heads
 // 19.3 -> 16.3; on the other side [2,20,2048,64] 62.2 -> 62.4, [1,8,4096,64]
 // 65.1 -> 69.5, [2,24,9216,64] x 512 keys 80.5 -> 89.3, [2,16,4096,64] 155 -> 164.
-// The rows of a head are addressed with 32-bit byte offsets.
+// The rows of a head, rounded up to whole chunks, are addressed with 32-bit byte
+// offsets.
 bool dense_rows_d64(const AttnArgs& a, int bh_count) {
-    auto addressable = [&](const View& x) { return x.st > 0 && x.st <= INT32_MAX / 2 / a.kv_tokens - 1; };
+    auto addressable = [&](const View& x) { return x.st > 0 && x.st <= INT32_MAX / 2 / ((int64_t)a.kv_blocks * kBlock + 1); };
     const int64_t chunks = (int64_t)bh_count * a.q_blocks * a.kv_blocks;
     return chunks < 13000 + 19 * (int64_t)bh_count * a.kv_blocks && addressable(a.k) && addressable(a.v);
 }

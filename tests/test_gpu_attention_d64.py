@@ -77,6 +77,21 @@ def test_rows_read_in_place_stay_inside_their_heads(native, head_dim, kv_tokens)
     assert bool((out[..., head_dim:] == 3.0).all())
 
 
+@pytest.mark.parametrize("head_dim", [64, 40])
+@pytest.mark.parametrize("kv_tokens", [1, 33, 65, 96, 130, 190])
+def test_rows_past_the_last_token_are_never_used(native, kv_tokens, head_dim):
+    """Keys and values of a longer buffer whose later rows (and later dims) are NaN."""
+    gen = torch.Generator().manual_seed(kv_tokens)
+    q = torch.randn((1, 2, 70, head_dim), generator=gen).to(torch.bfloat16)
+    k, v = (torch.full((1, 2, kv_tokens + 130, head_dim + 8), float("nan"), dtype=torch.bfloat16) for _ in range(2))
+    for t in (k, v):
+        t[:, :, :kv_tokens, :head_dim] = torch.randn((1, 2, kv_tokens, head_dim), generator=gen).to(torch.bfloat16)
+    k, v = (t.cuda()[:, :, :kv_tokens, :head_dim] for t in (k, v))
+    out = native.dense_attention(q.cuda(), k, v, head_dim ** -0.5)
+    expected = oatt.dense_attention(np32(q), np32(k), np32(v))
+    assert_close(np32(out), expected, 4 * UNIT[torch.bfloat16] * 5.0, 0.0, f"Tk={kv_tokens}")
+
+
 def test_dense_split_parts_of_very_different_scale(native):
     """Key parts whose maxima lie far apart (and rise along the list) merge without overflow or loss."""
     gen = torch.Generator().manual_seed(3)
