@@ -467,7 +467,7 @@ static int attend_impl(int32_t dtype, int32_t heads, int32_t tokens, int32_t hea
                        float scale, int32_t first_order, void* workspace, const StatsPlan& p, int bh, hipStream_t st) {
     const ForwardBuffers w = carve_forward(workspace, bh, tokens, head_dim, exact_blocks, 2);
     const pisa::TokenMap map = pisa::make_token_map(grid);
-    pisa::AttnArgs aa{};
+    pisa::AttnArgs aa;
     aa.q = to_view(q, heads);
     aa.o = to_out(out, heads);
     aa.kp = static_cast<const char*>(w.kp);
@@ -876,8 +876,6 @@ int attn_hip_dense_forward(int32_t dtype, int32_t batch, int32_t heads, int32_t 
     pisa::AttnArgs aa;
     memset(&aa, 0, sizeof(aa));
     aa.q = to_view(q, heads);
-    aa.k = to_view(k, heads);
-    aa.v = to_view(v, heads);
     aa.o = to_out(out, heads);
     aa.kp = kp;
     aa.vp = vp;
@@ -889,9 +887,10 @@ int attn_hip_dense_forward(int32_t dtype, int32_t batch, int32_t heads, int32_t 
     aa.scale_log2 = scale * pisa::kLog2e;
     aa.inv_scale_log2 = 1.0f / aa.scale_log2;
     aa.head_dim = head_dim;
-    if (padded == 64 && pisa::dense_rows_d64(aa, bh)) return pisa::launch_attention_d64_rows(dtype, aa, bh, st);
-    if ((rc = pisa::launch_kv_pack(dtype, padded, head_dim, aa.k, aa.v,
-                                   pisa::TokenMap{0, 0, 0}, kv_tokens, kv_blocks, bh, kp, vp, st)))
+    const pisa::KvRows kv{to_view(k, heads), to_view(v, heads)};
+    if (pisa::dense_rows_in_place(padded, aa, kv, bh)) return pisa::launch_attention_rows(dtype, padded, aa, kv, bh, st);
+    if ((rc = pisa::launch_kv_pack(dtype, padded, head_dim, kv.k, kv.v, pisa::TokenMap{0, 0, 0}, kv_tokens, kv_blocks, bh,
+                                   kp, vp, st)))
         return rc;
     return pisa::launch_attention(dtype, padded, false, false, aa, bh, st);
 }

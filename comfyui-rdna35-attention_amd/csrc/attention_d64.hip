@@ -1,5 +1,6 @@
 // Attention at head dims up to 64 (padded width 64): dense, and the PISA list
-// of selected blocks and centroids with the merge and first-order correction
+// of selected blocks and centroids with the merge and first-order correction;
+// and small dense calls at head dims up to 128, which read K and V in place
 // (attention.hip describes the computation; the operand tables, the transposed
 // scores and the lazy softmax are the same).
 #include "attention_softmax.hpp"
@@ -9,14 +10,10 @@ namespace pisa {
 
 namespace {
 
-constexpr int kD = 64;
-constexpr int KT = kD / 16;  // 16-deep k-steps of the score products
-constexpr int MD = kD / 32;  // 32-dim output tiles
-constexpr int NT = 2;        // 32-row query tiles of a 64-row block
-constexpr int kBlockBytes = kD * kBlock * 2;
+constexpr int NT = 2;  // 32-row query tiles of a 64-row block
 constexpr int kRawFlags = 0x00020000;  // untyped 32-bit buffer data format
 
-// Two waves per SIMD (256 registers each).  What bounds the loop, from
+// Width 64 runs two waves per SIMD (256 registers each).  What bounds the loop, from
 // register-only loops of its instruction mix (one MI355X, random operands):
 // per 32-key half chunk the 16 MFMAs hold the matrix core 512 cycles and the
 // vector issue port about 15 cycles each, the 94 ordinary softmax instructions
@@ -37,15 +34,21 @@ constexpr int kRawFlags = 0x00020000;  // untyped 32-bit buffer data format
 //
 // DIRECT (small dense calls): K and V are read from the caller's rows instead of
 // the packed tables, so no packing launch runs before.  The key operand is 16
-// bytes of one row per lane; of the values a lane reads two consecutive dims of
+// bytes of one row per lane; of the values a lane reads MD consecutive dims of
 // every key row it contracts (as in fixed_block_mfma_kernel), so output tile md
-// holds dims 2i + md of accumulator row i.  Each chunk costs more loads (20
-// instead of 8 per half, of 32 separate rows each): dense_rows_d64 says when
-// that is the better trade.
-template <typename T, bool SPARSE, bool TAIL, int W, bool DIRECT>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uint32_t* __restrict__ selmask) {
+// holds dims MD i + md of accumulator row i.  Each chunk costs more loads (at
+// width 64 20 instead of 8 per half, of 32 separate rows each):
+// dense_rows_in_place says when that is the better trade.  Width 128 exists in
+// this form only (340 registers, one wave per SIMD).
+template <typename T, int D, bool SPARSE, bool TAIL, int W, bool DIRECT>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 2 : 1, D <= 64 ? 2 : 1)))
+void attention_parts_kernel(AttnArgs a, KvRows kv, const int32_t* __restrict__ sel,
+                            const uint32_t* __restrict__ selmask) {
     static_assert(!DIRECT || (!SPARSE && !TAIL), "rows are read in place by the dense kernel only");
+    static_assert(D == 64 || (D == 128 && DIRECT), "packed tables of other widths: attention.hip");
+    constexpr int KT = D / 16;  // 16-deep k-steps of the score products
+    constexpr int MD = D / 32;  // 32-dim output tiles
+    constexpr int kBlockBytes = D * kBlock * 2;
     typedef typename Elem<T>::vec8 vec8;
     const int lane = threadIdx.x & 63;
     const int wave = W > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
@@ -109,24 +112,24 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
         (void*)(a.kp + (int64_t)bh * a.kv_blocks * kBlockBytes), (short)0, tab_bytes, kRawFlags);
     const __amdgpu_buffer_rsrc_t vp_rs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(a.vp + (int64_t)bh * a.kv_blocks * kBlockBytes), (short)0, tab_bytes, kRawFlags);
-    const int cen_bytes = TAIL ? a.npad * kD * 2 : 0;
+    const int cen_bytes = TAIL ? a.npad * D * 2 : 0;
     const __amdgpu_buffer_rsrc_t kc_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(TAIL ? a.kbar + (int64_t)bh * a.npad * kD * 2 : a.kp), (short)0, cen_bytes, kRawFlags);
+        (void*)(TAIL ? a.kbar + (int64_t)bh * a.npad * D * 2 : a.kp), (short)0, cen_bytes, kRawFlags);
     const __amdgpu_buffer_rsrc_t vc_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(TAIL ? a.vbar_t + (int64_t)bh * a.npad * kD * 2 : a.vp), (short)0, cen_bytes, kRawFlags);
+        (void*)(TAIL ? a.vbar_t + (int64_t)bh * a.npad * D * 2 : a.vp), (short)0, cen_bytes, kRawFlags);
     const int lane_off = lane * 16;
 
     // DIRECT: the rows of this head.  The whole byte offset of a load is its
     // vector offset, which the hardware checks against the size, so what lies
     // past the last row (or past its last dim) reads as zero.
-    const int k_row = DIRECT ? (int)a.k.st * 2 : 0, v_row = DIRECT ? (int)a.v.st * 2 : 0;  // bytes
+    const int k_row = DIRECT ? (int)kv.k.st * 2 : 0, v_row = DIRECT ? (int)kv.v.st * 2 : 0;  // bytes
     const __amdgpu_buffer_rsrc_t kr_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(DIRECT ? a.k.data + a.k.row(bh, 0) * 2 : a.kp), (short)0,
+        (void*)(DIRECT ? kv.k.data + kv.k.row(bh, 0) * 2 : a.kp), (short)0,
         DIRECT ? (a.kv_tokens - 1) * k_row + a.head_dim * 2 : 0, kRawFlags);
     const __amdgpu_buffer_rsrc_t vr_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(DIRECT ? a.v.data + a.v.row(bh, 0) * 2 : a.vp), (short)0,
+        (void*)(DIRECT ? kv.v.data + kv.v.row(bh, 0) * 2 : a.vp), (short)0,
         DIRECT ? (a.kv_tokens - 1) * v_row + a.head_dim * 2 : 0, kRawFlags);
-    const bool all_dims = a.head_dim >= kD;
+    const bool all_dims = a.head_dim >= D;
 
     auto is_tail = [&](int x) { return TAIL && min(x, n_chunks - 1) >= n_exact; };
     auto table_row = [&](int x) -> int {  // block id, or centroid chunk id; past the list, its last chunk again
@@ -142,7 +145,8 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
 
     vec8 kf[KT];     // key fragments of the half chunk scored next
     vec8 vf[DIRECT ? 1 : MD][2];  // value fragments of the half chunk multiplied next
-    uint32_t vr[DIRECT ? 2 : 1][8];  // DIRECT: dims 2col, 2col + 1 of its keys 16ss + 8(e/4) + 4half + e%4
+    // DIRECT: dims MD col .. + MD - 1 of its keys 16ss + 8(e/4) + 4half + e%4, two to a word
+    uint32_t vr[DIRECT ? 2 : 1][8][MD / 2];
     auto load_k = [&](bool tail, int row, int mt) {
         if constexpr (DIRECT) {
             const int off = (row * kBlock + mt * 32 + col) * k_row + half * 16;
@@ -156,13 +160,20 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
     };
     auto load_v = [&](bool tail, int row, int mt) {
         if constexpr (DIRECT) {
-            const int off = (row * kBlock + mt * 32 + 4 * half) * v_row + col * 4;
+            const int off = (row * kBlock + mt * 32 + 4 * half) * v_row + col * MD * 2;
 #pragma unroll
             for (int ss = 0; ss < 2; ++ss)
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    vr[ss][e] = __builtin_amdgcn_raw_buffer_load_b32(
-                        vr_rs, off + (16 * ss + 8 * (e >> 2) + (e & 3)) * v_row, 0, 0);
+                for (int e = 0; e < 8; ++e) {
+                    const int at = off + (16 * ss + 8 * (e >> 2) + (e & 3)) * v_row;
+                    if constexpr (MD == 2) {
+                        vr[ss][e][0] = __builtin_amdgcn_raw_buffer_load_b32(vr_rs, at, 0, 0);
+                    } else {
+                        const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(vr_rs, at, 0, 0);
+                        vr[ss][e][0] = x[0];
+                        vr[ss][e][MD / 2 - 1] = x[1];
+                    }
+                }
             return;
         }
 #pragma unroll
@@ -227,11 +238,12 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
 #pragma unroll
             for (int md = 0; md < MD; ++md) {
                 vec8 f;
-                if constexpr (DIRECT) {  // the 16-bit halves md of the 8 keys' words
+                if constexpr (DIRECT) {  // element md of the 8 keys
                     u32x4 w;
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        w[j] = __builtin_amdgcn_perm(vr[ss][2 * j + 1], vr[ss][2 * j], md ? 0x07060302u : 0x05040100u);
+                        w[j] = __builtin_amdgcn_perm(vr[ss][2 * j + 1][md / 2], vr[ss][2 * j][md / 2],
+                                                     md % 2 ? 0x07060302u : 0x05040100u);
                     f = __builtin_bit_cast(vec8, w);
                 } else {
                     f = vf[md][ss];
@@ -302,7 +314,9 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
         l[nt] = add_xor32(l[nt]);
         lt[nt] = add_xor32(lt[nt]);
     }
-    constexpr int kUnits = MD * NT * 2;  // (tile, pair of 4-row groups) output units, kUnits / W per wave
+    // output units, kUnits / W per wave: (tile, pair of 4-row accumulator groups), or
+    // DIRECT one group over all tiles (its 4 MD values are consecutive dims)
+    constexpr int kUnits = DIRECT ? NT * 4 : MD * NT * 2;
     __shared__ __attribute__((aligned(16))) float parts[W > 1 ? W * MD * NT * 16 * 64 : 4];
     __shared__ float stat[W > 1 ? W : 1][3][kBlock];
     if constexpr (W > 1) {
@@ -346,7 +360,7 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
     }
     const bool first_order = TAIL && a.ht != nullptr;
     const __amdgpu_buffer_rsrc_t ht_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(first_order ? a.ht + (int64_t)bh * kD * kD * 2 : a.kp), (short)0, first_order ? kD * kD * 2 : 0,
+        (void*)(first_order ? a.ht + (int64_t)bh * D * D * 2 : a.kp), (short)0, first_order ? D * D * 2 : 0,
         kRawFlags);
     typedef T vec4 __attribute__((ext_vector_type(4)));
     // 16-byte stores when every output row start is 16-byte aligned (8-byte ones otherwise)
@@ -356,11 +370,10 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
     for (int u = 0; u < kUnits / W; ++u) {
         // W = 1: tile and pair are constants and the accumulators stay in registers
         const int unit = wave * (kUnits / W) + u;
-        // DIRECT: unit = accumulator group g of query tile nt over both tiles md
-        // (dims 16g + 8half .. +7 of a lane's query)
         const int p = unit & 1, nt = DIRECT ? unit >> 2 : (unit >> 1) & 1, md = DIRECT ? 0 : unit >> 2;
         const bool second = nt != 0;
-        float x[8];
+        constexpr int kVals = DIRECT ? 4 * MD : 8;
+        float x[kVals];
         if constexpr (DIRECT) {
             const int g = unit & 3;
 #pragma unroll
@@ -395,7 +408,7 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
         const float lf = second ? l[1] : l[0];
         const float inv = 1.0f / lf;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] *= inv;
+        for (int e = 0; e < kVals; ++e) x[e] *= inv;
         if (first_order) {
             // rows 32md .. of the packed D x D matrix (kfrag_elem) times the query tile
             f32x16 corr;
@@ -411,22 +424,27 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
         const int tok = qbase + (second ? q_off[1] : q_off[0]);
         if (tok >= a.q_tokens) continue;  // lanes l and l + 32 (one query) take the same branch
         char* dst = a.o.data + a.o.row(bh, tok) * (int64_t)sizeof(T);
-        u32x2 w4[2];  // w4[g]: dims 32md + 8(2p + g) + 4half ..
+        u32x2 w4[kVals / 4];  // w4[g]: dims 32md + 8(2p + g) + 4half ..; DIRECT: MD (8g' + 4half) + 4g .. of group g'
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
+        for (int g = 0; g < kVals / 4; ++g) {
             vec4 out;
 #pragma unroll
             for (int e = 0; e < 4; ++e) out[e] = from_f32<T>(x[4 * g + e]);
             w4[g] = __builtin_bit_cast(u32x2, out);
         }
         if constexpr (DIRECT) {
-            const int d = 16 * (unit & 3) + 8 * half;
-            if (d >= a.head_dim) continue;
-            if (st16) {
-                *reinterpret_cast<u32x4*>(dst + d * sizeof(T)) = u32x4{w4[0][0], w4[0][1], w4[1][0], w4[1][1]};
-            } else {
-                *reinterpret_cast<u32x2*>(dst + d * sizeof(T)) = w4[0];
-                *reinterpret_cast<u32x2*>(dst + (d + 4) * sizeof(T)) = w4[1];
+#pragma unroll
+            for (int j = 0; j < MD / 2; ++j) {
+                const int d = MD * (8 * (unit & 3) + 4 * half) + 8 * j;
+                if (d >= a.head_dim) continue;
+                char* to = dst + d * sizeof(T);
+                if (st16) {
+                    *reinterpret_cast<u32x4*>(to) =
+                        u32x4{w4[2 * j][0], w4[2 * j][1], w4[2 * j + 1][0], w4[2 * j + 1][1]};
+                } else {
+                    *reinterpret_cast<u32x2*>(to) = w4[2 * j];
+                    *reinterpret_cast<u32x2*>(to + 8) = w4[2 * j + 1];
+                }
             }
             continue;
         }
@@ -461,7 +479,7 @@ void attention_d64_kernel(AttnArgs a, const int32_t* __restrict__ sel, const uin
 // grid that leaves SIMDs idle, or its last round nearly empty, is split; a full
 // one keeps one wave per block and merges nothing.  Eight waves use 134 KB of
 // LDS, one workgroup per CU, so nothing runs beside their merge.
-int waves_per_block(int64_t blocks, int n_chunks) {
+int waves_per_block(int64_t blocks, int n_chunks, int most) {
     static const int simds = [] {
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -472,7 +490,7 @@ int waves_per_block(int64_t blocks, int n_chunks) {
     if (simds <= 0) return 1;
     int best = 1;
     double least = 0.0;
-    for (int w = 1; w <= 8 && w <= n_chunks; w *= 2) {
+    for (int w = 1; w <= most && w <= n_chunks; w *= 2) {
         const double merge = w == 1 ? 1.0 : w == 8 ? 4.5 : 3.5;
         const double cost = (double)((blocks * w + simds - 1) / simds) * ((n_chunks + w - 1) / w + merge);
         if (w == 1 || cost < least) {
@@ -483,51 +501,70 @@ int waves_per_block(int64_t blocks, int n_chunks) {
     return best;
 }
 
-template <typename T, bool SPARSE, bool TAIL, bool DIRECT>
-int launch_t(const AttnArgs& a, int bh_count, hipStream_t stream) {
+template <typename T, int D, bool SPARSE, bool TAIL, bool DIRECT>
+int launch_t(const AttnArgs& a, const KvRows& kv, int bh_count, hipStream_t stream) {
     const int blocks = bh_count * a.q_blocks;
     const int n_chunks = (SPARSE ? a.exact : a.kv_blocks) + (TAIL ? a.npad / kBlock : 0);
-    const int w = waves_per_block(blocks, n_chunks);
-#define PISA_D64(W)                                                                                            \
-    hipLaunchKernelGGL((attention_d64_kernel<T, SPARSE, TAIL, W, DIRECT>), dim3(blocks), dim3(64 * W), 0, stream, a, \
-                       a.idx, a.selmask)
-    if (w == 1) PISA_D64(1);
-    else if (w == 2) PISA_D64(2);
-    else if (w == 4) PISA_D64(4);
-    else PISA_D64(8);
-#undef PISA_D64
-    return pisa_host::check_launch("attention_d64_kernel");
+    constexpr int kMost = D <= 64 ? 8 : 4;  // waves of a workgroup: two per SIMD, one at D = 128
+    const int w = waves_per_block(blocks, n_chunks, kMost);
+#define PISA_PARTS(W)                                                                                              \
+    hipLaunchKernelGGL((attention_parts_kernel<T, D, SPARSE, TAIL, W, DIRECT>), dim3(blocks), dim3(64 * W), 0, stream, \
+                       a, kv, a.idx, a.selmask)
+    if (w == 1) PISA_PARTS(1);
+    else if (w == 2) PISA_PARTS(2);
+    else if (w == 4) PISA_PARTS(4);
+    else if constexpr (kMost == 8) PISA_PARTS(8);
+#undef PISA_PARTS
+    return pisa_host::check_launch("attention_parts_kernel");
 }
 
 }  // namespace
 
 int launch_attention_d64(int dtype, bool sparse, const AttnArgs& a, int bh_count, hipStream_t stream) {
+    const KvRows none{};
     if (dtype == PISA_DTYPE_BF16)
-        return sparse ? launch_t<bf16_t, true, true, false>(a, bh_count, stream)
-                      : launch_t<bf16_t, false, false, false>(a, bh_count, stream);
-    return sparse ? launch_t<f16_t, true, true, false>(a, bh_count, stream)
-                  : launch_t<f16_t, false, false, false>(a, bh_count, stream);
+        return sparse ? launch_t<bf16_t, 64, true, true, false>(a, none, bh_count, stream)
+                      : launch_t<bf16_t, 64, false, false, false>(a, none, bh_count, stream);
+    return sparse ? launch_t<f16_t, 64, true, true, false>(a, none, bh_count, stream)
+                  : launch_t<f16_t, 64, false, false, false>(a, none, bh_count, stream);
 }
 
 // Reading rows in place saves the packing launch (about 4.5 us and 6.7 ns a key
 // block: 3.5 us for [1,8,1000,64], 11.3 us for [2,10,4096,64]) and costs 0.2 to
-// 0.4 ns for every chunk that a query block walks, so the line lies where
-// 0.35 ns x (query blocks x chunks) reaches it.  Packed -> in place, one MI355X:
-// [1,8,1000,64] 20.0 -> 16.9 us (host time of the launch included), [2,20,1024,64]
-// 30.1 -> 25.2, [2,10,2048,64] 45.9 -> 45.1, 64 keys of 4096 tokens in 32 heads
-// 19.3 -> 16.3; on the other side [2,20,2048,64] 62.2 -> 62.4, [1,8,4096,64]
-// 65.1 -> 69.5, [2,24,9216,64] x 512 keys 80.5 -> 89.3, [2,16,4096,64] 155 -> 164.
+// 0.4 ns for every chunk that a query block walks at width 64, more at 128, so
+// the line is one in (query blocks x chunks) and key blocks.  Packed -> in place,
+// us a call on one MI355X (small ones are bound by the host time of the launches):
+//   width 64:  [1,8,1000] 20.0 -> 16.9, [2,20,1024] 30.1 -> 25.2, [2,10,2048]
+//     45.9 -> 45.1, 64 keys of 4096 tokens in 32 heads 19.3 -> 16.3; past the line
+//     [2,20,2048] 62.2 -> 62.4, [1,8,4096] 65.1 -> 69.5, [2,24,9216] x 512 80 -> 89
+//   width 128: [1,8,1000] 22.1 -> 18.3, [1,10,1200] 36.8 -> 20.2, [1,8,2048]
+//     36.4 -> 28.6, [2,20,1024] 44.0 -> 39.2, [1,16,2048] 53.8 -> 50.4; past the line
+//     [1,24,2048] 68.5 -> 70.7, [2,16,4096] x 512 49.4 -> 58.6, [2,24,1536] 85 -> 102
+// Padded width 96 runs on the kernel of 128 (the dims past the head dim cost
+// products that a small call has to spare).  Its packed kernel neither splits a
+// block nor is persistent, so up to half a round of blocks the split wins at any
+// length: [1,8,2048,80] 44.5 -> 23.2, [1,8,4096,80] 87.2 -> 72.4, [1,2,9216,80]
+// 170 -> 137, [1,16,2048,96] 51.6 -> 40.5; past the line [1,24,2048,80]
+// 55.9 -> 61.2, [2,16,9216,80] x 256 51.4 -> 59.2.
 // The rows of a head, rounded up to whole chunks, are addressed with 32-bit byte
 // offsets.
-bool dense_rows_d64(const AttnArgs& a, int bh_count) {
+bool dense_rows_in_place(int padded, const AttnArgs& a, const KvRows& kv, int bh_count) {
+    if (padded > 128) return false;
     auto addressable = [&](const View& x) { return x.st > 0 && x.st <= INT32_MAX / 2 / ((int64_t)a.kv_blocks * kBlock + 1); };
-    const int64_t chunks = (int64_t)bh_count * a.q_blocks * a.kv_blocks;
-    return chunks < 13000 + 19 * (int64_t)bh_count * a.kv_blocks && addressable(a.k) && addressable(a.v);
+    if (!addressable(kv.k) || !addressable(kv.v)) return false;
+    const int64_t blocks = (int64_t)bh_count * a.q_blocks, tables = (int64_t)bh_count * a.kv_blocks;
+    const int64_t chunks = blocks * a.kv_blocks;
+    if (padded == 64) return chunks < 13000 + 19 * tables;
+    if (padded == 96) return blocks <= 512 || chunks < 7000 + 20 * tables;
+    return chunks < 9500 + 14 * tables;
 }
 
-int launch_attention_d64_rows(int dtype, const AttnArgs& a, int bh_count, hipStream_t stream) {
-    return dtype == PISA_DTYPE_BF16 ? launch_t<bf16_t, false, false, true>(a, bh_count, stream)
-                                    : launch_t<f16_t, false, false, true>(a, bh_count, stream);
+int launch_attention_rows(int dtype, int padded, const AttnArgs& a, const KvRows& kv, int bh_count, hipStream_t stream) {
+    if (padded == 64)
+        return dtype == PISA_DTYPE_BF16 ? launch_t<bf16_t, 64, false, false, true>(a, kv, bh_count, stream)
+                                        : launch_t<f16_t, 64, false, false, true>(a, kv, bh_count, stream);
+    return dtype == PISA_DTYPE_BF16 ? launch_t<bf16_t, 128, false, false, true>(a, kv, bh_count, stream)
+                                    : launch_t<f16_t, 128, false, false, true>(a, kv, bh_count, stream);
 }
 
 }  // namespace pisa

@@ -138,7 +138,6 @@ struct RouteArgs {
 
 struct AttnArgs {
     View q;
-    View k, v;        // the caller's rows (launch_attention_d64_rows only)
     OutView o;
     const char* kp;   // [BH][kv_blocks] packed key blocks (kfrag_elem order)
     const char* vp;   // [BH][kv_blocks] packed value blocks (vfrag_elem order)
@@ -204,10 +203,13 @@ int launch_attention(int dtype, int padded, bool sparse, bool tail, const AttnAr
                      hipStream_t stream);
 // The same at padded width 64, dense or PISA (attention_d64.hip).
 int launch_attention_d64(int dtype, bool sparse, const AttnArgs& a, int bh_count, hipStream_t stream);
-// Small dense calls at that width read K and V where they are (a.k, a.v; no
-// packed tables): whether a call is one, and its launch.
-bool dense_rows_d64(const AttnArgs& a, int bh_count);
-int launch_attention_d64_rows(int dtype, const AttnArgs& a, int bh_count, hipStream_t stream);
+// Small dense calls at padded widths 64 and 128 read K and V where they are
+// instead of packed tables: whether a call is one, and its launch.
+struct KvRows {
+    View k, v;
+};
+bool dense_rows_in_place(int padded, const AttnArgs& a, const KvRows& kv, int bh_count);
+int launch_attention_rows(int dtype, int padded, const AttnArgs& a, const KvRows& kv, int bh_count, hipStream_t stream);
 // Packed key / value blocks of width `padded` (dims >= head_dim and rows >= kv_tokens are zero);
 // block j row r is token map(64 j + r).
 int launch_kv_pack(int dtype, int padded, int head_dim, const View& k, const View& v, TokenMap map, int kv_tokens,

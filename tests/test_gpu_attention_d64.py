@@ -1,4 +1,5 @@
-"""The head-dim-64 attention kernel on the MI355X at the sizes where its key split changes.
+"""The split-list attention kernel (head dim 64, and small dense calls up to 128) on the MI355X at the sizes where
+its key split and its choice between packed tables and rows in place change.
 
 One to eight waves share a query block and merge their parts of its chunk list; the split follows the number of
 query blocks and chunks, so the shapes below reach every split, ragged last blocks, lists shorter than the split
@@ -41,7 +42,15 @@ def native():
     (20, 1600, 512, 64),    # 500 blocks of 8 chunks: two waves
     (64, 1024, 130, 64),    # 1024 blocks: one wave
     (2, 64, 449, 8),        # eight waves on eight chunks, one each
+    (3, 130, 1000, 128),    # head dims up to 128 in place: four waves
+    (2, 65, 77, 120),       # two chunks
+    (40, 500, 500, 104),    # 320 blocks of 8 chunks: two waves
+    (64, 1100, 64, 128),    # one chunk: one wave
+    (1, 200, 700, 80),      # padded width 96 on the wider kernel
+    (5, 6400, 640, 96),     # 500 blocks
     # the shapes above read K and V in place, these from packed tables
+    (32, 4096, 512, 96),
+    (16, 4096, 1279, 128),
     (1, 7990, 8000, 64),    # 125 blocks of 125 chunks: eight waves
     (2, 6400, 6400, 40),    # 200 blocks: four waves
     (5, 6400, 2500, 64),    # 500 blocks of 40 chunks: two waves
@@ -58,7 +67,7 @@ def test_dense_splits_match_oracle(native, dtype, heads, q_tokens, kv_tokens, he
     assert_close(np32(out[:, :, rows]), expected, atol, 0.0, f"dense {heads}x{q_tokens}x{kv_tokens} D={head_dim}")
 
 
-@pytest.mark.parametrize("head_dim,kv_tokens", [(64, 130), (40, 257), (8, 64)])
+@pytest.mark.parametrize("head_dim,kv_tokens", [(64, 130), (40, 257), (8, 64), (128, 130), (112, 257), (80, 65)])
 def test_rows_read_in_place_stay_inside_their_heads(native, head_dim, kv_tokens):
     """Views into one fused [B,T,3,H,D+8] tensor whose other elements are NaN: nothing past a row or past the last
     token reaches the result, an infinite value in the last row stays one column's, and stores end with the row."""
@@ -77,7 +86,7 @@ def test_rows_read_in_place_stay_inside_their_heads(native, head_dim, kv_tokens)
     assert bool((out[..., head_dim:] == 3.0).all())
 
 
-@pytest.mark.parametrize("head_dim", [64, 40])
+@pytest.mark.parametrize("head_dim", [64, 40, 128, 104, 72])
 @pytest.mark.parametrize("kv_tokens", [1, 33, 65, 96, 130, 190])
 def test_rows_past_the_last_token_are_never_used(native, kv_tokens, head_dim):
     """Keys and values of a longer buffer whose later rows (and later dims) are NaN."""
