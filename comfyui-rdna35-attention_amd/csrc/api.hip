@@ -829,6 +829,21 @@ int pisa_hip_fuse_spatial_epilogue(int32_t dtype, int32_t batch, int32_t heads, 
                               batch * heads, static_cast<hipStream_t>(stream));
 }
 
+// Whether the bytes from a view's first element to its last can touch another
+// view's (a negative stride counts as touching).
+static bool views_touch(const pisa_view& a, int32_t a_tokens, const pisa_view& b, int32_t b_tokens, int32_t batch,
+                        int32_t heads, int32_t head_dim) {
+    auto bytes = [&](const pisa_view& v, int32_t tokens) -> int64_t {
+        if (v.batch_stride < 0 || v.head_stride < 0 || v.token_stride < 0) return -1;
+        return 2 * ((batch - 1) * v.batch_stride + (heads - 1) * v.head_stride + (tokens - 1) * v.token_stride + head_dim);
+    };
+    const int64_t na = bytes(a, a_tokens), nb = bytes(b, b_tokens);
+    if (na < 0 || nb < 0) return true;
+    const char* pa = static_cast<const char*>(a.data);
+    const char* pb = static_cast<const char*>(b.data);
+    return pa < pb + nb && pb < pa + na;
+}
+
 int64_t attn_hip_dense_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens, int32_t head_dim) {
     if (batch <= 0 || heads <= 0 || kv_tokens <= 0 || head_dim <= 0 || !sizes_fit(batch, heads, kv_tokens)) return 0;
     const int64_t blocks = (kv_tokens + pisa::kBlock - 1) / pisa::kBlock;
@@ -888,7 +903,11 @@ int attn_hip_dense_forward(int32_t dtype, int32_t batch, int32_t heads, int32_t 
     aa.inv_scale_log2 = 1.0f / aa.scale_log2;
     aa.head_dim = head_dim;
     const pisa::KvRows kv{to_view(k, heads), to_view(v, heads)};
-    if (pisa::dense_rows_in_place(padded, aa, kv, bh)) return pisa::launch_attention_rows(dtype, padded, aa, kv, bh, st);
+    // (an output over the keys or values is written only after the packed tables hold them)
+    if (pisa::dense_rows_in_place(padded, aa, kv, bh) &&
+        !views_touch(out, q_tokens, k, kv_tokens, batch, heads, head_dim) &&
+        !views_touch(out, q_tokens, v, kv_tokens, batch, heads, head_dim))
+        return pisa::launch_attention_rows(dtype, padded, aa, kv, bh, st);
     if ((rc = pisa::launch_kv_pack(dtype, padded, head_dim, kv.k, kv.v, pisa::TokenMap{0, 0, 0}, kv_tokens, kv_blocks, bh,
                                    kp, vp, st)))
         return rc;

@@ -86,6 +86,22 @@ def test_rows_read_in_place_stay_inside_their_heads(native, head_dim, kv_tokens)
     assert bool((out[..., head_dim:] == 3.0).all())
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("target", ["k", "v"])
+def test_output_over_the_keys_or_values(native, head_dim, target):
+    """An output stored over K or V: the call then packs them first instead of reading them while it stores.
+
+    4096 query blocks, more than fit the GPU at once: without the packing, late blocks would read stored outputs.
+    """
+    gen = torch.Generator().manual_seed(9)
+    q, rows = (torch.randn((2, 32, 4096, head_dim), generator=gen).to(torch.bfloat16).cuda() for _ in range(2))
+    other = torch.randn((2, 32, 64, head_dim), generator=gen).to(torch.bfloat16).cuda()
+    k, v = (rows[:, :, :64], other) if target == "k" else (other, rows[:, :, :64])
+    expected = native.dense_attention(q, k, v, head_dim ** -0.5)
+    native._launch_dense(q, k, v, rows, head_dim ** -0.5)
+    assert_close(np32(rows), np32(expected), 4 * UNIT[torch.bfloat16] * 5.0, 0.0, f"out over {target}")
+
+
 @pytest.mark.parametrize("head_dim", [64, 40, 128, 104, 72])
 @pytest.mark.parametrize("kv_tokens", [1, 33, 65, 96, 130, 190])
 def test_rows_past_the_last_token_are_never_used(native, kv_tokens, head_dim):
