@@ -1,6 +1,7 @@
 // Exact attention on bf16/fp16 MFMA with the PISA tail, first-order
 // correction and merge fused into the epilogue (padded head dims above 64;
-// attention_d64.hip holds the kernel of the narrower ones).
+// attention_d64.hip holds the kernel of the narrower ones and of small dense
+// calls at head dims up to 128).
 //
 // One wavefront owns one 64-row query block (all four SIMDs of a CU run
 // independent query blocks, 1 wave per SIMD, up to 512 registers each; at
