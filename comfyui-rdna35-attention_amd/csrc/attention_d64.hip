@@ -106,17 +106,20 @@ void attention_parts_kernel(AttnArgs a, KvRows kv, const int32_t* __restrict__ s
     const int hi = (wave + 1) * n_chunks / W;
     const int32_t* my_idx = SPARSE ? sel + ((int64_t)bh * a.q_blocks + qb) * a.exact : nullptr;
     const uint32_t* my_mask = TAIL ? selmask + ((int64_t)bh * a.q_blocks + qb) * a.mask_words : nullptr;
-    // packed tables of this head as buffer resources (reads past a table return zero)
+    // Packed tables of this head as buffer resources (reads past a table return
+    // zero).  Exact or centroid chunk is a choice between base pointers and
+    // sizes, which stay in scalar registers; a choice between resources would go
+    // through private memory, with a wait for every load in flight.
     const int tab_bytes = a.kv_blocks * kBlockBytes;
-    const __amdgpu_buffer_rsrc_t kp_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(a.kp + (int64_t)bh * a.kv_blocks * kBlockBytes), (short)0, tab_bytes, kRawFlags);
-    const __amdgpu_buffer_rsrc_t vp_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(a.vp + (int64_t)bh * a.kv_blocks * kBlockBytes), (short)0, tab_bytes, kRawFlags);
     const int cen_bytes = TAIL ? a.npad * D * 2 : 0;
-    const __amdgpu_buffer_rsrc_t kc_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(TAIL ? a.kbar + (int64_t)bh * a.npad * D * 2 : a.kp), (short)0, cen_bytes, kRawFlags);
-    const __amdgpu_buffer_rsrc_t vc_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(TAIL ? a.vbar_t + (int64_t)bh * a.npad * D * 2 : a.vp), (short)0, cen_bytes, kRawFlags);
+    const char* const kp = a.kp + (int64_t)bh * tab_bytes;
+    const char* const vp = a.vp + (int64_t)bh * tab_bytes;
+    const char* const kc = TAIL ? a.kbar + (int64_t)bh * cen_bytes : kp;
+    const char* const vc = TAIL ? a.vbar_t + (int64_t)bh * cen_bytes : vp;
+    auto table = [&](bool tail, const char* exact, const char* centroids) {
+        return __builtin_amdgcn_make_buffer_rsrc((void*)(TAIL && tail ? centroids : exact), (short)0,
+                                                 TAIL && tail ? cen_bytes : tab_bytes, kRawFlags);
+    };
     const int lane_off = lane * 16;
 
     // DIRECT: the rows of this head.  The whole byte offset of a load is its
@@ -137,7 +140,7 @@ void attention_parts_kernel(AttnArgs a, KvRows kv, const int32_t* __restrict__ s
         if (TAIL && x >= n_exact) return x - n_exact;
         return SPARSE ? my_idx[x] : x;
     };
-    auto ld_frag = [&](const __amdgpu_buffer_rsrc_t& rs, int off, int frag) -> vec8 {
+    auto ld_frag = [&](__amdgpu_buffer_rsrc_t rs, int off, int frag) -> vec8 {
         const int soff = __builtin_amdgcn_readfirstlane(off + (frag >> 2) * 4096);
         return __builtin_bit_cast(vec8,
                                   __builtin_amdgcn_raw_buffer_load_b128(rs, lane_off + (frag & 3) * 1024, soff, 0));
@@ -155,8 +158,9 @@ void attention_parts_kernel(AttnArgs a, KvRows kv, const int32_t* __restrict__ s
                 kf[t] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(kr_rs, off + t * 32, 0, 0));
             return;
         }
+        const __amdgpu_buffer_rsrc_t rs = table(tail, kp, kc);
 #pragma unroll
-        for (int t = 0; t < KT; ++t) kf[t] = ld_frag(tail ? kc_rs : kp_rs, row * kBlockBytes, mt * KT + t);
+        for (int t = 0; t < KT; ++t) kf[t] = ld_frag(rs, row * kBlockBytes, mt * KT + t);
     };
     auto load_v = [&](bool tail, int row, int mt) {
         if constexpr (DIRECT) {
@@ -176,11 +180,11 @@ void attention_parts_kernel(AttnArgs a, KvRows kv, const int32_t* __restrict__ s
                 }
             return;
         }
+        const __amdgpu_buffer_rsrc_t rs = table(tail, vp, vc);
 #pragma unroll
         for (int md = 0; md < MD; ++md)
 #pragma unroll
-            for (int ss = 0; ss < 2; ++ss)
-                vf[md][ss] = ld_frag(tail ? vc_rs : vp_rs, row * kBlockBytes, md * 4 + 2 * mt + ss);
+            for (int ss = 0; ss < 2; ++ss) vf[md][ss] = ld_frag(rs, row * kBlockBytes, md * 4 + 2 * mt + ss);
     };
     // Centroid chunks get their score bias (log2 of the block's length over c,
     // -inf for selected blocks and padding) from one more MFMA per query tile:

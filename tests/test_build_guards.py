@@ -19,6 +19,12 @@ register allocator rebuilt a spilled query fragment inside the chunk loop
 with one of its four dwords taken from the previous iteration's scores (the
 head-dim 256 kernel, whose query fragments now live in LDS instead).
 
+A fifth guard: the attention kernels load through buffer resources held in
+scalar registers.  A resource that the compiler takes from private memory (a
+choice between two of them by reference) or holds in vector registers costs a
+wait for every load in flight and a loop over the lanes' values around each
+load.
+
 These tests compile the sources to gfx950 assembly with the library's own
 flags (about a minute) and fail with the offending lines if any of this stops
 holding.
@@ -104,6 +110,18 @@ def test_no_kernel_spills_vector_registers(device_asm):
                 spills.append(f"{name}: {kernel} spills {count} registers")
     assert checked >= 40, f"kernel metadata of only {checked} kernels found"
     assert not spills, "\n".join(spills)
+
+
+def test_attention_buffer_resources_stay_in_scalar_registers(device_asm):
+    checked = 0
+    for source in ("attention.hip", "attention_dense.hip", "attention_d64.hip"):
+        for name, body in _kernels(device_asm[source]).items():
+            loops = [i for i, instr in enumerate(body) if instr.startswith("s_cbranch_execnz")]
+            loads = [i for i, instr in enumerate(body) if instr.startswith("buffer_load")]
+            checked += bool(loads)
+            around = [i for i in loads if any(0 < end - i <= 6 for end in loops)]
+            assert not around, f"{source}: {name} loops over lanes around {len(around)} buffer loads"
+    assert checked >= 40, f"buffer loads in only {checked} attention kernels"
 
 
 def test_only_the_lds_copies_use_m0(device_asm):
