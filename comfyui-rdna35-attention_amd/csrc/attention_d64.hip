@@ -419,8 +419,14 @@ void attention_parts_kernel(AttnArgs a, KvRows kv, const int32_t* __restrict__ s
 #pragma unroll
             for (int v = 0; v < 16; ++v) corr[v] = 0.0f;
 #pragma unroll
-            for (int t = 0; t < KT; ++t)
-                corr = mfma32(ld_frag(ht_rs, md * KT * 1024, t), second ? qreg[1][t] : qreg[0][t], corr);
+            for (int t = 0; t < KT; ++t) {
+                // element by element: a choice between the arrays' elements puts them in private memory
+                const u32x4 q0 = __builtin_bit_cast(u32x4, qreg[0][t]), q1 = __builtin_bit_cast(u32x4, qreg[1][t]);
+                u32x4 qt;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) qt[j] = second ? q1[j] : q0[j];
+                corr = mfma32(ld_frag(ht_rs, md * KT * 1024, t), __builtin_bit_cast(vec8, qt), corr);
+            }
             const float wa = (second ? lt[1] : lt[0]) * inv * a.corr_scale;
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[e] += (p ? corr[8 + e] : corr[e]) * wa;

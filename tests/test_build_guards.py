@@ -25,6 +25,10 @@ choice between two of them by reference) or holds in vector registers costs a
 wait for every load in flight and a loop over the lanes' values around each
 load.
 
+A sixth: no kernel has private memory at all.  An array whose index the
+compiler does not know (query fragments chosen by the wave's number) goes there
+without any register being counted as spilled.
+
 These tests compile the sources to gfx950 assembly with the library's own
 flags (about a minute) and fail with the offending lines if any of this stops
 holding.
@@ -110,6 +114,20 @@ def test_no_kernel_spills_vector_registers(device_asm):
                 spills.append(f"{name}: {kernel} spills {count} registers")
     assert checked >= 40, f"kernel metadata of only {checked} kernels found"
     assert not spills, "\n".join(spills)
+
+
+def test_no_kernel_has_private_memory(device_asm):
+    private, checked = [], 0
+    for name, asm in device_asm.items():
+        if "amdhsa.kernels:" not in asm:  # host-only source (api.hip)
+            continue
+        entries = asm.split("amdhsa.kernels:", 1)[1]
+        for kernel, size in re.findall(r"\.name:\s+(\S+)[^-]*?\.private_segment_fixed_size:\s+(\d+)", entries, re.S):
+            checked += 1
+            if int(size):
+                private.append(f"{name}: {kernel} has {size} bytes per lane")
+    assert checked >= 40, f"kernel metadata of only {checked} kernels found"
+    assert not private, "\n".join(private)
 
 
 def test_attention_buffer_resources_stay_in_scalar_registers(device_asm):
