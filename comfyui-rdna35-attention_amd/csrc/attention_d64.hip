@@ -282,23 +282,27 @@ void attention_parts_kernel(AttnArgs a, KvRows kv, const int32_t* __restrict__ s
     // its second half, then the second half's beside the scores of the next
     // chunk.  `last` (no next chunk) and `plain` (this chunk and the next are
     // exact full blocks) are constants of each inlined copy.
-    auto chunk_step = [&](int cc, bool last, bool plain) __attribute__((always_inline)) {
+    auto chunk_step = [&](int cc, bool last, bool plain, bool half0_only) __attribute__((always_inline)) {
         const int row2 = (plain && !SPARSE) ? cc + 2 : table_row(cc + 2);
         const bool t0 = !plain && is_tail(cc), t1 = !plain && !last && is_tail(cc + 1);
         vec8 pf[NT][2];
-        scores(sb, t0, row0, 1);
+        if (!half0_only) scores(sb, t0, row0, 1);
         if (!last) load_k(t1, row1, 0);
         probs_half<T, NT>(sa, c, nm, l, lt, t0, pf);
         pv(pf);
-        load_v(t0, row0, 1);
-        check(sb, t0, row0, 1, plain);
+        if (!half0_only) {
+            load_v(t0, row0, 1);
+            check(sb, t0, row0, 1, plain);
+        }
 
         if (!last) {
             scores(sa, t1, row1, 0);
             load_k(t1, row1, 1);
         }
-        probs_half<T, NT>(sb, c, nm, l, lt, t0, pf);
-        pv(pf);
+        if (!half0_only) {
+            probs_half<T, NT>(sb, c, nm, l, lt, t0, pf);
+            pv(pf);
+        }
         if (!last) {
             load_v(t1, row1, 0);
             check(sa, t1, row1, 0, plain);
@@ -308,9 +312,11 @@ void attention_parts_kernel(AttnArgs a, KvRows kv, const int32_t* __restrict__ s
     };
     // the selection is ascending, so only the last exact chunk can be short
     int cc = lo;
-    for (; cc + 3 <= n_exact && cc + 1 < hi; ++cc) chunk_step(cc, false, true);
-    for (; cc + 1 < hi; ++cc) chunk_step(cc, false, false);
-    chunk_step(cc, true, false);
+    for (; cc + 3 <= n_exact && cc + 1 < hi; ++cc) chunk_step(cc, false, true, false);
+    for (; cc + 1 < hi; ++cc) chunk_step(cc, false, false, false);
+    // A last centroid chunk whose second half is only padding ends after its
+    // first (the rest would add exactly zero to l, l_tail and O).
+    chunk_step(cc, true, false, TAIL && hi == n_chunks && row0 * kBlock + 32 >= a.centroids);
 
     // ---- merge of the W parts, first-order correction, store
 #pragma unroll

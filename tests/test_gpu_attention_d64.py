@@ -138,6 +138,11 @@ def test_dense_split_parts_of_very_different_scale(native):
     (2, 500, 7, True, 0.125),     # all but one block exact, short last block
     (1, 4100, 6, True, 0.125),    # two centroid chunks, the second nearly all padding
     (16, 1024, 4, False, 1e-3),   # a small softmax scale: bias / scale beyond fp16's range
+    # the last centroid chunk's second half: only padding (skipped), or one centroid
+    (33, 2048, 0, True, 0.125),   # one wave: 32 centroids
+    (32, 2103, 3, True, 0.125),   # one wave: 33
+    (16, 2043, 9, True, 0.125),   # two waves: 32
+    (1, 4140, 20, True, 0.125),   # eight waves: 65, one in the second chunk
 ])
 def test_sparse_splits_match_oracle(native, dtype, heads, tokens, exact, first_order, scale):
     gen = torch.Generator().manual_seed(tokens + exact)
