@@ -71,10 +71,11 @@ def _in_place_views(q, k, v, layout: str, heads: int | None):
     None sends the call through normalize_qkv_to_bh_t_d: flat [BH,T,D] tensors, every malformed call (it reports
     them), fake or subclassed tensors (tracing) and storage whose rows the kernels could only read element by
     element (it makes the contiguous copy).  On contiguous tensors the two ways run the same kernel on the same
-    rows; on the others this one reads in place what the other copies first.
+    rows; on the others this one reads in place what the other copies first.  A tensor that requires grad always takes
+    the other way: with grad mode off its copy does not require grad (the kernel runs), while a view of it still does.
     """
     if type(q) is not torch.Tensor or type(k) is not torch.Tensor or type(v) is not torch.Tensor or \
-            torch.compiler.is_compiling():
+            torch.compiler.is_compiling() or q.requires_grad or k.requires_grad or v.requires_grad:
         return None
     shape = q.shape
     if k.shape != shape or v.shape != shape or not q.is_cuda or not q.numel():

@@ -79,3 +79,25 @@ def test_rows_readable_needs_unit_stride_and_aligned_rows():
     assert dispatch._rows_readable(torch.zeros((B, H, T, D + 4), dtype=torch.float32)[..., :D])
     assert not dispatch._rows_readable(torch.zeros(B * H * T * D + 1, dtype=torch.bfloat16)[1:].view(B, H, T, D))
     assert dispatch._in_place_views(x, x, x, "bhtd", None) is None  # CPU tensors take the eager route
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["bhtd", "bthd"])
+def test_strided_inputs_that_require_grad_run_the_kernel_with_grad_mode_off(layout):
+    """Their contiguous copies do not require grad; with grad mode on the call is the eager path's."""
+    gen = torch.Generator().manual_seed(13)
+    x = torch.randn((B, T, 3 * H * D), generator=gen).to(torch.bfloat16).cuda().requires_grad_()
+    plain = x.detach()
+
+    def call(t):
+        q, k, v = t.chunk(3, dim=2)
+        if layout == "bhtd":
+            q, k, v = (p.view(B, T, H, D).transpose(1, 2) for p in (q, k, v))
+        return fixed_block_attention(q, k, v, layout=layout, heads=H, return_diagnostics=True)
+
+    for off in (torch.no_grad, torch.inference_mode):
+        with off():
+            out, info = call(x)
+        assert info["backend"] == "hip" and torch.equal(out, call(plain)[0])
+    _, info = call(x)
+    assert info["fallback_reason"] == "requires_grad_uses_reference"
