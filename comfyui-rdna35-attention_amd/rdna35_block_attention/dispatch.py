@@ -58,10 +58,17 @@ def _hip_reject_reason(q_flat: torch.Tensor, k_flat: torch.Tensor, v_flat: torch
 
 
 def _rows_readable(tensor: torch.Tensor) -> bool:
-    """Unit head_dim stride and every row 16-byte aligned: the rows the matrix-core kernels read where they are."""
+    """Unit head_dim stride and every row 16-byte aligned: the rows the matrix-core kernels read where they are.
+
+    False for tensors without storage (torch.func transforms wrap theirs in plain tensors of that kind).
+    """
+    try:
+        address = tensor.data_ptr()
+    except RuntimeError:
+        return False
     strides = tensor.stride()
     unit = 16 // tensor.element_size()
-    return strides[3] == 1 and tensor.data_ptr() % 16 == 0 and \
+    return strides[3] == 1 and address % 16 == 0 and \
         not (strides[0] % unit or strides[1] % unit or strides[2] % unit)
 
 

@@ -101,3 +101,19 @@ def test_strided_inputs_that_require_grad_run_the_kernel_with_grad_mode_off(layo
         assert info["backend"] == "hip" and torch.equal(out, call(plain)[0])
     _, info = call(x)
     assert info["fallback_reason"] == "requires_grad_uses_reference"
+
+
+def test_tensors_wrapped_by_a_transform_are_not_readable():
+    x = torch.zeros((2, B, H, T, D))
+    assert torch.func.vmap(lambda t: t.sum() * dispatch._rows_readable(t))(x).tolist() == [0.0, 0.0]
+
+
+@pytest.mark.gpu
+def test_vmap_of_a_call_the_kernel_does_not_take():
+    """Head dim 48 falls back to the eager path, under vmap as outside it."""
+    gen = torch.Generator().manual_seed(14)
+    q, k, v = (torch.randn((2, B, H, T, 48), generator=gen).cuda() for _ in range(3))
+    out = torch.func.vmap(lambda *qkv: fixed_block_attention(*qkv, layout="bhtd"))(q, k, v)
+    for i in range(2):
+        expected = fixed_block_attention(q[i], k[i], v[i], layout="bhtd")
+        torch.testing.assert_close(out[i], expected, atol=1e-5, rtol=1e-5)  # fp32 products in another batching
