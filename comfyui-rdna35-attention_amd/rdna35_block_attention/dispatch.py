@@ -72,7 +72,7 @@ def _rows_readable(tensor: torch.Tensor) -> bool:
         not (strides[0] % unit or strides[1] % unit or strides[2] % unit)
 
 
-def _in_place_views(q, k, v, layout: str, heads: int | None):
+def _in_place_views(q, k, v, layout: str, heads: int | None, mask=None):
     """(q, k, v as [B,H,T,D] views, LayoutInfo) of plain tensors the kernels can read where they are, else None.
 
     None sends the call through normalize_qkv_to_bh_t_d: flat [BH,T,D] tensors, every malformed call (it reports
@@ -80,7 +80,10 @@ def _in_place_views(q, k, v, layout: str, heads: int | None):
     element (it makes the contiguous copy).  On contiguous tensors the two ways run the same kernel on the same
     rows; on the others this one reads in place what the other copies first.  A tensor that requires grad always takes
     the other way: with grad mode off its copy does not require grad (the kernel runs), while a view of it still does.
+    So does a call with a subclassed mask, which runs as the registered op.
     """
+    if mask is not None and type(mask) is not torch.Tensor:
+        return None
     if type(q) is not torch.Tensor or type(k) is not torch.Tensor or type(v) is not torch.Tensor or \
             torch.compiler.is_compiling() or q.requires_grad or k.requires_grad or v.requires_grad:
         return None
@@ -115,7 +118,7 @@ def fixed_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, 
                   return_diagnostics=return_diagnostics)
     if mode == "reference":
         return _fallback(q, k, v, reason="mode_reference", **common)
-    in_place = _in_place_views(q, k, v, layout, heads)
+    in_place = _in_place_views(q, k, v, layout, heads, mask)
     if in_place is not None:
         (q4, k4, v4), info = in_place
     else:

@@ -117,3 +117,18 @@ def test_vmap_of_a_call_the_kernel_does_not_take():
     for i in range(2):
         expected = fixed_block_attention(q[i], k[i], v[i], layout="bhtd")
         torch.testing.assert_close(out[i], expected, atol=1e-5, rtol=1e-5)  # fp32 products in another batching
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["bhtd", "bthd"])
+def test_a_subclassed_mask_gives_its_type_to_the_result(layout):
+    class Mask(torch.Tensor):
+        pass
+
+    gen = torch.Generator().manual_seed(15)
+    shape = (B, H, T, D) if layout == "bhtd" else (B, T, H * D)
+    q, k, v = (torch.randn(shape, generator=gen).cuda() for _ in range(3))
+    mask = (torch.rand((T, T), generator=gen) < 0.8).cuda()
+    out = fixed_block_attention(q, k, v, layout=layout, heads=H, mask=mask.as_subclass(Mask))
+    assert type(out) is Mask
+    assert torch.equal(out.as_subclass(torch.Tensor), fixed_block_attention(q, k, v, layout=layout, heads=H, mask=mask))
