@@ -1,7 +1,8 @@
 // Exact attention on bf16/fp16 MFMA with the PISA tail, first-order
-// correction and merge fused into the epilogue (padded head dims above 64;
-// attention_d64.hip holds the kernel of the narrower ones and of small dense
-// calls at head dims up to 128).
+// correction and merge fused into the epilogue (padded head dims above 64, and
+// dense calls of 64 that give each SIMD at most one wave; attention_d64.hip
+// holds the kernel of the other narrow ones and of small dense calls at head
+// dims up to 128).
 //
 // One wavefront owns one 64-row query block (all four SIMDs of a CU run
 // independent query blocks, 1 wave per SIMD, up to 512 registers each; at
@@ -915,8 +916,8 @@ int launch_attention_t(const AttnArgs& a_in, int bh_count, hipStream_t stream) {
 // chunk loop better and the sparse one worse.  This file without the macro
 // holds the sparse kernels, the dispatcher and the packing kernel.
 #define PISA_DENSE_INSTANCES(X) \
-    X(bf16_t, 96) X(bf16_t, 128) X(bf16_t, 160) X(bf16_t, 192) X(bf16_t, 256) \
-    X(f16_t, 96) X(f16_t, 128) X(f16_t, 160) X(f16_t, 192) X(f16_t, 256)
+    X(bf16_t, 64) X(bf16_t, 96) X(bf16_t, 128) X(bf16_t, 160) X(bf16_t, 192) X(bf16_t, 256) \
+    X(f16_t, 64) X(f16_t, 96) X(f16_t, 128) X(f16_t, 160) X(f16_t, 192) X(f16_t, 256)
 #ifdef PISA_ATTENTION_DENSE
 #define PISA_DENSE_INSTANCE(T, D) template int launch_attention_t<T, D, false, false>(const AttnArgs&, int, hipStream_t);
 PISA_DENSE_INSTANCES(PISA_DENSE_INSTANCE)
@@ -937,6 +938,9 @@ int launch_attention_d(bool sparse, bool tail, const AttnArgs& a, int bh_count, 
 template <typename T>
 int launch_attention_dt(int padded, bool sparse, bool tail, const AttnArgs& a, int bh_count, hipStream_t stream) {
     switch (padded) {
+        case 64:
+            if (sparse || tail) return pisa_host::fail(PISA_ERR_UNSUPPORTED, "attention kernel: head dim 64 is dense only here");
+            return launch_attention_t<T, 64, false, false>(a, bh_count, stream);
         case 96: return launch_attention_d<T, 96>(sparse, tail, a, bh_count, stream);
         case 128: return launch_attention_d<T, 128>(sparse, tail, a, bh_count, stream);
         case 160: return launch_attention_d<T, 160>(sparse, tail, a, bh_count, stream);
@@ -948,7 +952,8 @@ int launch_attention_dt(int padded, bool sparse, bool tail, const AttnArgs& a, i
 
 int launch_attention(int dtype, int padded, bool sparse, bool tail, const AttnArgs& a, int bh_count,
                      hipStream_t stream) {
-    if (padded == 64 && sparse == tail) return launch_attention_d64(dtype, sparse, a, bh_count, stream);
+    if (padded == 64 && sparse == tail && (sparse || !dense_d64_one_wave(a, bh_count)))
+        return launch_attention_d64(dtype, sparse, a, bh_count, stream);
     if (dtype == PISA_DTYPE_BF16) return launch_attention_dt<bf16_t>(padded, sparse, tail, a, bh_count, stream);
     return launch_attention_dt<f16_t>(padded, sparse, tail, a, bh_count, stream);
 }

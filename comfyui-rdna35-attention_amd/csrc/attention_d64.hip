@@ -486,6 +486,18 @@ void attention_parts_kernel(AttnArgs a, KvRows kv, const int32_t* __restrict__ s
     }
 }
 
+// SIMDs of the device (0 if it does not say).
+int simd_count() {
+    static const int simds = [] {
+        int dev = 0, cus = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            return 0;
+        return 4 * cus;
+    }();
+    return simds;
+}
+
 // Waves per query block: the W with the smallest estimate of
 //     rounds of the SIMDs x (chunks of one wave + the chunk times a merge costs),
 // which follows the measured times (1280 blocks of 64 chunks, [2,10,4096,64]:
@@ -496,13 +508,7 @@ void attention_parts_kernel(AttnArgs a, KvRows kv, const int32_t* __restrict__ s
 // one keeps one wave per block and merges nothing.  Eight waves use 134 KB of
 // LDS, one workgroup per CU, so nothing runs beside their merge.
 int waves_per_block(int64_t blocks, int n_chunks, int most) {
-    static const int simds = [] {
-        int dev = 0, cus = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            return 0;
-        return 4 * cus;
-    }();
+    const int simds = simd_count();
     if (simds <= 0) return 1;
     int best = 1;
     double least = 0.0;
@@ -535,6 +541,19 @@ int launch_t(const AttnArgs& a, const KvRows& kv, int bh_count, hipStream_t stre
 }
 
 }  // namespace
+
+// At most one wave per SIMD, from packed tables: nothing then hides the loads of
+// the kernel above, and the one of attention.hip, whose 264 registers hold both
+// halves' fragments, is the faster one.  Call times, this kernel -> that one:
+// [1,14,2880,64] 57.4 -> 54.5 us, 2048 keys of 4096 tokens in 12 heads 41.1 ->
+// 39.3, [1,11,4630,64] 86.8 -> 82.6, [1,8,8192,64] 150.3 -> 146.7, [1,32,2048,64]
+// 52.0 -> 51.2.  Splits and grids of more than a round stay here ([1,16,2048,64],
+// two waves per block, 39.0 against 39.5; 2808 blocks of 11 chunks 48.7 against
+// 50.2).
+bool dense_d64_one_wave(const AttnArgs& a, int bh_count) {
+    const int64_t blocks = (int64_t)bh_count * a.q_blocks;
+    return blocks <= simd_count() && waves_per_block(blocks, a.kv_blocks, 8) == 1;
+}
 
 int launch_attention_d64(int dtype, bool sparse, const AttnArgs& a, int bh_count, hipStream_t stream) {
     const KvRows none{};

@@ -201,7 +201,9 @@ int launch_stats_means(int dtype, int padded, const StatsArgs& a, int bh_count, 
 // `padded` = padded_head_dim(a.head_dim); dense (sparse = tail = false) or PISA (both true).
 int launch_attention(int dtype, int padded, bool sparse, bool tail, const AttnArgs& a, int bh_count,
                      hipStream_t stream);
-// The same at padded width 64, dense or PISA (attention_d64.hip).
+// The same at padded width 64, dense or PISA (attention_d64.hip), except dense
+// calls of at most one wave per SIMD.
+bool dense_d64_one_wave(const AttnArgs& a, int bh_count);
 int launch_attention_d64(int dtype, bool sparse, const AttnArgs& a, int bh_count, hipStream_t stream);
 // Small dense calls at padded widths 64 and 128 read K and V where they are
 // instead of packed tables: whether a call is one, and its launch.
