@@ -565,22 +565,32 @@ int launch_attention_d64(int dtype, bool sparse, const AttnArgs& a, int bh_count
 }
 
 // Reading rows in place saves the packing launch (about 4.5 us and 6.7 ns a key
-// block: 3.5 us for [1,8,1000,64], 11.3 us for [2,10,4096,64]) and costs 0.2 to
-// 0.4 ns for every chunk that a query block walks at width 64, more at 128, so
-// the line is one in (query blocks x chunks) and key blocks.  Packed -> in place,
-// us a call on one MI355X (small ones are bound by the host time of the launches):
-//   width 64:  [1,8,1000] 20.0 -> 16.9, [2,20,1024] 30.1 -> 25.2, [2,10,2048]
-//     45.9 -> 45.1, 64 keys of 4096 tokens in 32 heads 19.3 -> 16.3; past the line
-//     [2,20,2048] 62.2 -> 62.4, [1,8,4096] 65.1 -> 69.5, [2,24,9216] x 512 80 -> 89
-//   width 128: [1,8,1000] 22.1 -> 18.3, [1,10,1200] 36.8 -> 20.2, [1,8,2048]
-//     36.4 -> 28.6, [2,20,1024] 44.0 -> 39.2, [1,16,2048] 53.8 -> 50.4; past the line
-//     [1,24,2048] 68.5 -> 70.7, [2,16,4096] x 512 49.4 -> 58.6, [2,24,1536] 85 -> 102
-// Padded width 96 runs on the kernel of 128 (the dims past the head dim cost
-// products that a small call has to spare).  Its packed kernel neither splits a
-// block nor is persistent, so up to half a round of blocks the split wins at any
-// length: [1,8,2048,80] 44.5 -> 23.2, [1,8,4096,80] 87.2 -> 72.4, [1,2,9216,80]
-// 170 -> 137, [1,16,2048,96] 51.6 -> 40.5; past the line [1,24,2048,80]
-// 55.9 -> 61.2, [2,16,9216,80] x 256 51.4 -> 59.2.
+// block at width 64) and costs 0.05 to 0.1 us, more at 128, for every chunk that
+// the busiest CU walks: `load` below, which a grid of a few blocks, or of a few
+// blocks over a whole round, makes larger than its share of all chunks.  So the
+// lines are in `load` and key blocks (`tables`), one for each kernel that the
+// packed call would run and each way the rows lie in memory, under bounds in all
+// chunks.  They were fitted to the device times of 130 calls of 2 to 48 heads in
+// three layouts ([B,H,T,D], [B,T,H,D] and a fused projection) at head dims 40, 64,
+// 80, 96, 104 and 128 on one MI355X.  Packed / in place, us:
+//   width 64, at most one wave per SIMD (dense_d64_one_wave, the better packed
+//     kernel of the two): [1,24,2048,64] 43.1 / 42.7, 2048 keys of 4096 tokens in
+//     12 heads 39.4 / 42.7; as [B,T,H,D] rows [1,24,1536,64] 33.5 / 36.4 and at
+//     head dim 40 [1,24,2048] 41.9 / 47.1.  Otherwise [1,16,2048,64] 39.0 / 36.6,
+//     16384 keys of 256 tokens in 2 heads 67.6 / 78.6, [2,24,9216,64] x 77
+//     34.9 / 33.6.
+//   width 128 splits small grids where the packed kernel does not.  Up to a
+//     quarter of a round in place always wins ([1,8,2048,128] 35.1 / 28.5); up to
+//     half a round it wins against the kernel of uneven grids ([2,15,940,128]
+//     39.3 / 28.5), and against the persistent one the more of the SIMDs its two
+//     waves per block fill ([1,16,2048,128] 51.9 / 49.8, [2,8,1374,128] 33.1 /
+//     35.9, [1,8,3072,128] 57.2 / 69.9); above, its chunks cost half as much again
+//     ([1,16,9216,128] x 256 38.9 / 46.8, [2,20,1024,128] 42.2 / 38.7).
+//   padded width 96 runs on the kernel of 128 in place, and on one that neither
+//     splits nor persists packed: [1,8,4096,80] 84.9 / 70.7, [1,24,1536,80]
+//     42.6 / 45.9.  Rows that are not whole 128-byte lines but lie a multiple of
+//     them apart ([B,T,H,D] with 8 heads of 80) cost a quarter more each:
+//     [1,8,3072,80] 65.4 / 69.2, against 75.0 / 65.1 for [1,7,3373,80].
 // The rows of a head, rounded up to whole chunks, are addressed with 32-bit byte
 // offsets.
 bool dense_rows_in_place(int padded, const AttnArgs& a, const KvRows& kv, int bh_count) {
@@ -589,9 +599,24 @@ bool dense_rows_in_place(int padded, const AttnArgs& a, const KvRows& kv, int bh
     if (!addressable(kv.k) || !addressable(kv.v)) return false;
     const int64_t blocks = (int64_t)bh_count * a.q_blocks, tables = (int64_t)bh_count * a.kv_blocks;
     const int64_t chunks = blocks * a.kv_blocks;
-    if (padded == 64) return chunks < 13000 + 19 * tables;
-    if (padded == 96) return blocks <= 512 || chunks < 7000 + 20 * tables;
-    return chunks < 9500 + 14 * tables;
+    const int64_t simds = simd_count() > 0 ? simd_count() : 1024;
+    const int64_t load = (blocks + simds / 4 - 1) / (simds / 4) * a.kv_blocks;
+    const bool joined = kv.k.st == a.head_dim && kv.v.st == a.head_dim;  // one row right after the other
+    if (padded == 64) {
+        if (chunks >= 13000 + 19 * tables) return false;
+        if (dense_d64_one_wave(a, bh_count))
+            return 100 * load < (a.head_dim < 64 ? 1300 + 5 * tables : joined ? 4600 + 7 * tables : 1400 + 7 * tables);
+        return waves_per_block(blocks, a.kv_blocks, 8) == 1 || 200 * load < 6000 + 27 * tables;
+    }
+    if (padded == 128 ? chunks >= 9500 + 14 * tables : blocks > simds / 2 && chunks >= 7000 + 20 * tables) return false;
+    if (blocks <= simds / 4) return true;
+    const bool persistent = a.head_dim == 128 && blocks % 8 == 0;  // the packed kernel (launch_attention_t)
+    if (blocks <= simds / 2) {
+        const bool lines_apart = a.head_dim % 64 != 0 && (kv.k.st % 64 == 0 || kv.v.st % 64 == 0);
+        return !(persistent || lines_apart) || 100 * load < 600 + 23 * tables * blocks / simds;
+    }
+    if (padded == 96) return 100 * load < 800 + (joined ? 8 : 4) * tables;
+    return 200 * load < 2400 + (joined && a.head_dim < 128 ? 40 : persistent ? 13 : 16) * tables;
 }
 
 int launch_attention_rows(int dtype, int padded, const AttnArgs& a, const KvRows& kv, int bh_count, hipStream_t stream) {

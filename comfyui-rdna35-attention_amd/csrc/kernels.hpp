@@ -205,7 +205,7 @@ int launch_attention(int dtype, int padded, bool sparse, bool tail, const AttnAr
 // calls of at most one wave per SIMD.
 bool dense_d64_one_wave(const AttnArgs& a, int bh_count);
 int launch_attention_d64(int dtype, bool sparse, const AttnArgs& a, int bh_count, hipStream_t stream);
-// Small dense calls at padded widths 64 and 128 read K and V where they are
+// Small dense calls at padded widths 64, 96 and 128 read K and V where they are
 // instead of packed tables: whether a call is one, and its launch.
 struct KvRows {
     View k, v;

@@ -54,11 +54,11 @@ def native():
     (1, 7990, 8000, 64),    # 125 blocks of 125 chunks: eight waves
     (2, 6400, 6400, 40),    # 200 blocks: four waves
     (5, 6400, 2500, 64),    # 500 blocks of 40 chunks: two waves
+    (25, 2650, 2600, 64),   # 1050 blocks of 41 chunks: four waves, five rounds
     # at most one wave per SIMD: the 512-register kernel
     (16, 4096, 1279, 64),   # 1024 blocks of 20 chunks
     (12, 4090, 2010, 40),   # 768 of 32, padded dims, short last rows and keys
     (14, 2880, 2880, 64),   # 630 of 45
-    (25, 2650, 2600, 64),   # 1050 of 41: two waves' rounds
 ])
 def test_dense_splits_match_oracle(native, dtype, heads, q_tokens, kv_tokens, head_dim):
     gen = torch.Generator().manual_seed(heads * 7 + q_tokens + kv_tokens)
