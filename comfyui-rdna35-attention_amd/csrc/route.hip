@@ -64,8 +64,10 @@ __device__ __forceinline__ f32x4 mfma16_f32(float a, float b, f32x4 c) {
 // to LDS (rows past TILE are formed and not used).  Selection: wave w takes
 // rows TILE/4 w .. TILE/4 (w+1) - 1 together, lane l reading candidates l,
 // l+64, ... of a row from LDS.  T: dtype of the H_sum copy of the fused
-// reduction workgroups.
-template <int PL, int TILE, typename T>  // candidates per lane in the selection: N <= 64 * PL
+// reduction workgroups.  PT > 0: fp32 means of exactly 64 PT dims, read as whole
+// rows (launch_route_t); in a kernel of its own, since beside this path the
+// general loop ran 1 to 4 % slower at the other head dims.
+template <int PL, int TILE, typename T, int PT>  // candidates per lane in the selection: N <= 64 * PL
 __global__ __launch_bounds__(64 * kRouteWaves) void route_topk_kernel(RouteArgs a, ReduceArgs r, int fuse_reduce) {
     static_assert(TILE == 16 || TILE == 8, "routing rows per workgroup");
     constexpr int kRouteTile = TILE;
@@ -172,7 +174,52 @@ __global__ __launch_bounds__(64 * kRouteWaves) void route_topk_kernel(RouteArgs 
             for (int v = 0; v < 4; ++v) acc[v] = 0.0f;
         }
     };
-    if (a.qc_bf16 && a.kc_pack && D == 128) {
+    if constexpr (PT > 0) {
+        // The general loop's products in its order (bit-identical scores), with
+        // the query operands in registers for all tiles and the next tile's
+        // whole key rows in flight: half the loads, and no address or piece
+        // arithmetic between the MFMAs.  The launch takes 97 -> 70 us at 40
+        // heads x 512 blocks x 128 dims and 22.9 -> 19.2 us at 32 x 256 x 64
+        // (8-row workgroups there: 21.2).  Two rows' registers fit the 128 that
+        // four workgroups per CU leave up to 128 dims only.
+        auto load_row = [&](const float* row, f32x4 (&f)[4 * PT]) {
+#pragma unroll
+            for (int st = 0; st < 4 * PT; ++st) f[st] = *reinterpret_cast<const f32x4*>(row + 16 * st + 4 * kg);
+        };
+        auto load_tile = [&](int m, f32x4 (&kf)[4 * PT]) {
+            const int j = min((wave + kRouteWaves * min(m, my_tiles - 1)) * 16 + c16, N - 1);
+            load_row(kbase + (int64_t)j * (64 * PT), kf);
+        };
+        f32x4 qf[4 * PT], kt[2][4 * PT];
+        load_row(qrow, qf);
+        if (rnd) {
+#pragma unroll
+            for (int st = 0; st < 4 * PT; ++st)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) qf[st][e] = round_bf16(qf[st][e]);
+        }
+        auto tile = [&](int m, const f32x4 (&kf)[4 * PT]) {
+            f32x4 c4 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int st = 0; st < 4 * PT; ++st)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) c4 = mfma16_f32(qf[st][e], rnd ? round_bf16(kf[st][e]) : kf[st][e], c4);
+            const int j = (wave + kRouteWaves * m) * 16 + c16;
+            if (j < N) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) s_lds[(4 * kg + v) * stride + j] = c4[v];
+            }
+        };
+        if (my_tiles > 0) {
+            load_tile(0, kt[0]);
+            for (int m = 0; m < my_tiles; m += 2) {
+                load_tile(m + 1, kt[1]);
+                tile(m, kt[0]);
+                load_tile(m + 2, kt[0]);
+                tile(m + 1, kt[1]);
+            }
+        }
+    } else if (a.qc_bf16 && a.kc_pack && D == 128) {
         // bf16 means (HYD, bf16 inputs): 16x16x32 bf16 MFMA, lane (kg, c16)
         // holding dims 32s + 8kg .. +7 of query row i0 + c16 (A) and of centroid
         // ct*16 + c16 (B) for step s; products are exact, sums fp32.  All loads
@@ -209,56 +256,6 @@ __global__ __launch_bounds__(64 * kRouteWaves) void route_topk_kernel(RouteArgs 
                 tile(m + 1, kt[1]);
             }
         }
-    } else if (D == 64 || D == 128) {
-        // The general loop's products in its order (bit-identical scores), with
-        // the query operands in registers for all tiles and the next tile's
-        // whole key rows in flight: half the loads, and no address or piece
-        // arithmetic between the MFMAs.  The launch takes 107 -> 80 us at 40
-        // heads x 512 blocks x 128 dims and 23.2 -> 19.6 us at 32 x 256 x 64
-        // (kernel traces; 8-row workgroups there: 21.2).  Two rows' registers
-        // fit the 128 that four workgroups per CU leave up to 128 dims only.
-        auto whole_rows = [&](auto pieces_of_row) {
-            constexpr int PT = decltype(pieces_of_row)::value;
-            auto load_row = [&](const float* row, f32x4 (&f)[4 * PT]) {
-#pragma unroll
-                for (int st = 0; st < 4 * PT; ++st) f[st] = *reinterpret_cast<const f32x4*>(row + 16 * st + 4 * kg);
-            };
-            auto load_tile = [&](int m, f32x4 (&kf)[4 * PT]) {
-                const int j = min((wave + kRouteWaves * min(m, my_tiles - 1)) * 16 + c16, N - 1);
-                load_row(kbase + (int64_t)j * (64 * PT), kf);
-            };
-            f32x4 qf[4 * PT], kt[2][4 * PT];
-            load_row(qrow, qf);
-            if (rnd) {
-#pragma unroll
-                for (int st = 0; st < 4 * PT; ++st)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) qf[st][e] = round_bf16(qf[st][e]);
-            }
-            auto tile = [&](int m, const f32x4 (&kf)[4 * PT]) {
-                f32x4 c4 = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int st = 0; st < 4 * PT; ++st)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) c4 = mfma16_f32(qf[st][e], rnd ? round_bf16(kf[st][e]) : kf[st][e], c4);
-                const int j = (wave + kRouteWaves * m) * 16 + c16;
-                if (j < N) {
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) s_lds[(4 * kg + v) * stride + j] = c4[v];
-                }
-            };
-            if (my_tiles > 0) {
-                load_tile(0, kt[0]);
-                for (int m = 0; m < my_tiles; m += 2) {
-                    load_tile(m + 1, kt[1]);
-                    tile(m, kt[0]);
-                    load_tile(m + 2, kt[0]);
-                    tile(m + 1, kt[1]);
-                }
-            }
-        };
-        if (D == 64) whole_rows(std::integral_constant<int, 1>{});
-        else whole_rows(std::integral_constant<int, 2>{});
     } else {
     if (pieces > 0) {
         // every step loads and multiplies (a piece index past the wave's last
@@ -363,7 +360,7 @@ __global__ __launch_bounds__(64 * kRouteWaves) void route_topk_kernel(RouteArgs 
     }
 }
 
-template <int PL, int TILE, typename T>
+template <int PL, int TILE, typename T, int PT>
 static int launch_route_pl(const RouteArgs& a, const ReduceArgs& r, int fuse, hipStream_t stream) {
     const int row_tiles = (a.blocks + TILE - 1) / TILE;
     const int bh_count = a.rows / a.blocks;
@@ -382,7 +379,7 @@ static int launch_route_pl(const RouteArgs& a, const ReduceArgs& r, int fuse, hi
     if (lds_limit <= 0 || lds + static_lds > (size_t)lds_limit)
         return pisa_host::fail(PISA_ERR_UNSUPPORTED, "routing over %d blocks needs %zu bytes of LDS, device allows %d",
                                a.blocks, lds + static_lds, lds_limit);
-    hipLaunchKernelGGL((route_topk_kernel<PL, TILE, T>), grid, dim3(64 * kRouteWaves), lds, stream, a, r, fuse);
+    hipLaunchKernelGGL((route_topk_kernel<PL, TILE, T, PT>), grid, dim3(64 * kRouteWaves), lds, stream, a, r, fuse);
     return PISA_OK;
 }
 
@@ -392,7 +389,7 @@ static int launch_route_pl(const RouteArgs& a, const ReduceArgs& r, int fuse, hi
 // tiles of all N candidates, so at C5 (N = 512, 1280 workgroups of 16 rows)
 // halving the rows per workgroup doubles that work and the launch is 65 us
 // slower.
-template <typename T>
+template <typename T, int PT>
 static int launch_route_t(const RouteArgs& a, const ReduceArgs& r, int fuse, hipStream_t stream) {
     static const int cus = [] {
         int dev = 0, n = 0;
@@ -404,23 +401,41 @@ static int launch_route_t(const RouteArgs& a, const ReduceArgs& r, int fuse, hip
     const int pl = (a.blocks + 63) / 64;
     const int64_t wgs16 = (int64_t)(a.rows / a.blocks) * ((a.blocks + 15) / 16);
     const bool rows8 = pl <= 4 && wgs16 < 2 * (int64_t)cus;
-    if (pl <= 1) return rows8 ? launch_route_pl<1, 8, T>(a, r, fuse, stream) : launch_route_pl<1, 16, T>(a, r, fuse, stream);
-    if (pl <= 2) return rows8 ? launch_route_pl<2, 8, T>(a, r, fuse, stream) : launch_route_pl<2, 16, T>(a, r, fuse, stream);
-    if (pl <= 3) return rows8 ? launch_route_pl<3, 8, T>(a, r, fuse, stream) : launch_route_pl<3, 16, T>(a, r, fuse, stream);
-    if (pl <= 4) return rows8 ? launch_route_pl<4, 8, T>(a, r, fuse, stream) : launch_route_pl<4, 16, T>(a, r, fuse, stream);
-    if (pl <= 8) return launch_route_pl<8, 16, T>(a, r, fuse, stream);
-    return launch_route_pl<16, 16, T>(a, r, fuse, stream);
+    if constexpr (PT != 2) {  // (PT = 2: more than 64 blocks)
+        if (pl <= 1)
+            return rows8 ? launch_route_pl<1, 8, T, PT>(a, r, fuse, stream) : launch_route_pl<1, 16, T, PT>(a, r, fuse, stream);
+    }
+    if (pl <= 2) return rows8 ? launch_route_pl<2, 8, T, PT>(a, r, fuse, stream) : launch_route_pl<2, 16, T, PT>(a, r, fuse, stream);
+    if (pl <= 3) return rows8 ? launch_route_pl<3, 8, T, PT>(a, r, fuse, stream) : launch_route_pl<3, 16, T, PT>(a, r, fuse, stream);
+    if (pl <= 4) return rows8 ? launch_route_pl<4, 8, T, PT>(a, r, fuse, stream) : launch_route_pl<4, 16, T, PT>(a, r, fuse, stream);
+    if (pl <= 8) return launch_route_pl<8, 16, T, PT>(a, r, fuse, stream);
+    return launch_route_pl<16, 16, T, PT>(a, r, fuse, stream);
+}
+
+// Whole rows (PT) at 64 dims, and at 128 where a wave has more than one score
+// tile: with one (up to 64 blocks) nothing is in flight beside the first row's
+// loads and the general loop, which starts on half a row, is faster (8 heads x
+// 16 / 64 / 80 / 128 blocks x 128 dims: 4.9 / 6.6 / 8.6 / 9.5 us general, 5.9 /
+// 6.9 / 7.6 / 8.1 whole; x 64 dims: 5.0 / 6.6 / 7.3 general, 4.7 / 5.3 / 6.0).
+template <typename T>
+static int launch_route_d(const RouteArgs& a, const ReduceArgs& r, int fuse, hipStream_t stream) {
+    const bool bf16_means = a.qc_bf16 && a.kc_pack;
+    if constexpr (std::is_same<T, bf16_t>::value) {  // 64 dims: never fused
+        if (a.head_dim == 64) return launch_route_t<T, 1>(a, r, fuse, stream);
+    }
+    if (a.head_dim == 128 && !bf16_means && a.blocks > 64) return launch_route_t<T, 2>(a, r, fuse, stream);
+    return launch_route_t<T, 0>(a, r, fuse, stream);
 }
 
 int launch_route(const RouteArgs& a, hipStream_t stream) {
     ReduceArgs none{};
-    if (int rc = launch_route_t<bf16_t>(a, none, 0, stream)) return rc;
+    if (int rc = launch_route_d<bf16_t>(a, none, 0, stream)) return rc;
     return pisa_host::check_launch("route_topk_kernel");
 }
 
 int launch_route_reduce(int dtype, const RouteArgs& a, const ReduceArgs& r, hipStream_t stream) {
     if (a.head_dim != 128) return pisa_host::fail(PISA_ERR_UNSUPPORTED, "fused H_sum reduction needs head dim 128");
-    const int rc = dtype == PISA_DTYPE_BF16 ? launch_route_t<bf16_t>(a, r, 1, stream) : launch_route_t<f16_t>(a, r, 1, stream);
+    const int rc = dtype == PISA_DTYPE_BF16 ? launch_route_d<bf16_t>(a, r, 1, stream) : launch_route_d<f16_t>(a, r, 1, stream);
     if (rc) return rc;
     return pisa_host::check_launch("route_topk_kernel");
 }

@@ -1,4 +1,5 @@
-"""Routing scores at head dims 64 and 128, whose rows the kernel holds and loads whole, on the MI355X.
+"""Routing scores at head dims 64 and 128, whose rows the kernel holds and loads whole (at 128 above 64 blocks), on the
+MI355X.
 
 The same centroids with 16 zero dims appended take the general loop over the row, which forms the same products in the
 same order and adds zeros, so scores and selections must be equal bit for bit.  Against a float64 product the fp32 sums
@@ -14,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("round_bf16", [False, True])
 @pytest.mark.parametrize("head_dim", [64, 128])
-@pytest.mark.parametrize("blocks", [1, 15, 16, 17, 63, 65, 81, 129, 256, 257, 513, 1024])
+@pytest.mark.parametrize("blocks", [1, 15, 16, 17, 63, 64, 65, 81, 129, 256, 257, 513, 1024])
 def test_whole_row_scores_equal_the_general_loop(blocks, head_dim, round_bf16):
     import mi355x_pisa
 
