@@ -745,18 +745,18 @@ void attention_persistent_kernel(AttnArgs a, const int32_t* __restrict__ sel, co
 // ---- packed key and value blocks (kfrag_elem / vfrag_elem order at the
 // padded width D; dims >= d_real and rows >= kv_tokens are zero; block j
 // row r is token map(64 j + r)).  One workgroup per block: 64 rows x D of K
-// and V are read with 16-byte loads (kRows rows per thread, two at D = 64 so
-// that all 256 threads load), the key fragments are written straight from
-// registers and the value block is transposed through LDS.
+// and V are read with 16-byte loads (four rows per thread, so at D = 64 half of
+// the threads load), the key fragments are written straight from registers and
+// the value block is transposed through LDS.
 //
 // MEANS (generic PISA off head dim 128): the same pass reads the query rows
 // too and forms the block means q_bar, k_bar, v_bar (fp32 sums over a thread's
 // rows, then over the row groups in order, divided by the block's length), so
 // K and V are read once for both: [1,32,16384,64] 49 + 49 us as two kernels,
-// 56-58 us as one for 335 MB (63 with four rows per thread, which leaves half
-// the threads of D = 64 idle).  K and V are then read with the non-temporal
-// hint (nothing reads those rows again, and the tables written here stay in the
-// caches for the attention kernel: call 733 -> 724 us).
+// 56-58 us as one for 335 MB.  At D = 64 it takes two rows per thread, so that
+// all 256 threads load (63 us with four).  K and V are then read with the
+// non-temporal hint (nothing reads those rows again, and the tables written here
+// stay in the caches for the attention kernel: call 733 -> 724 us).
 template <typename T, int D, bool MEANS>
 __global__ __launch_bounds__(256) void kv_pack_kernel(View k, View v, TokenMap map, int kv_tokens, int kv_blocks,
                                                       int d_real, char* kp, char* vp, PackMeans m) {

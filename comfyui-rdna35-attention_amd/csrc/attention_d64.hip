@@ -2,7 +2,8 @@
 // of selected blocks and centroids with the merge and first-order correction;
 // and small dense calls at head dims up to 128, which read K and V in place
 // (attention.hip describes the computation; the operand tables, the transposed
-// scores and the lazy softmax are the same).
+// scores and the lazy softmax are the same; it also runs the dense packed calls
+// that give each SIMD at most one wave, dense_d64_one_wave).
 #include "attention_softmax.hpp"
 #include "kernels.hpp"
 
@@ -37,9 +38,9 @@ constexpr int kRawFlags = 0x00020000;  // untyped 32-bit buffer data format
 // bytes of one row per lane; of the values a lane reads MD consecutive dims of
 // every key row it contracts (as in fixed_block_mfma_kernel), so output tile md
 // holds dims MD i + md of accumulator row i.  Each chunk costs more loads (at
-// width 64 20 instead of 8 per half, of 32 separate rows each):
-// dense_rows_in_place says when that is the better trade.  Width 128 exists in
-// this form only (340 registers, one wave per SIMD).
+// width 64 20 instead of 8 per half: 4 of keys, from 32 rows each, and 16 of
+// values, from two rows each): dense_rows_in_place says when that is the better
+// trade.  Width 128 exists in this form only (340 registers, one wave per SIMD).
 template <typename T, int D, bool SPARSE, bool TAIL, int W, bool DIRECT>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 2 : 1, D <= 64 ? 2 : 1)))
 void attention_parts_kernel(AttnArgs a, KvRows kv, const int32_t* __restrict__ sel,

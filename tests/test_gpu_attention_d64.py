@@ -41,7 +41,7 @@ def native():
     (40, 300, 1024, 64),    # 200 blocks: four waves
     (20, 1600, 512, 64),    # 500 blocks of 8 chunks: two waves
     (64, 1024, 130, 64),    # 1024 blocks: one wave
-    (2, 64, 449, 8),        # eight waves on eight chunks, one each
+    (2, 64, 449, 8),        # eight chunks, the last of one key: four waves
     (3, 130, 1000, 128),    # head dims up to 128 in place: four waves
     (2, 65, 77, 120),       # two chunks
     (40, 500, 500, 104),    # 320 blocks of 8 chunks: two waves
@@ -139,8 +139,8 @@ def test_dense_split_parts_of_very_different_scale(native):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("heads,tokens,exact,first_order,scale", [
     (2, 1000, 0, False, 0.125),   # centroids only: one chunk, one wave
-    (2, 500, 7, True, 0.125),     # all but one block exact, short last block
-    (1, 4100, 6, True, 0.125),    # two centroid chunks, the second nearly all padding
+    (2, 500, 7, True, 0.125),     # all but one block exact, short last block: four waves
+    (1, 4100, 6, True, 0.125),    # two centroid chunks, the second nearly all padding: four waves
     (16, 1024, 4, False, 1e-3),   # a small softmax scale: bias / scale beyond fp16's range
     # the last centroid chunk's second half: only padding (skipped), or one centroid
     (33, 2048, 0, True, 0.125),   # one wave: 32 centroids
