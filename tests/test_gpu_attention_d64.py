@@ -136,6 +136,25 @@ def test_dense_split_parts_of_very_different_scale(native):
     assert_close(np32(out), expected, atol, 0.0, "rising scores")
 
 
+@pytest.mark.parametrize("heads,q_tokens,kv_tokens,head_dim", [
+    (1, 70, 832, 64), (1, 70, 512, 128),  # in place: eight waves of one or two chunks, four of two
+    (2, 256, 16384, 64),                  # packed: eight waves of 32
+])
+def test_dense_parts_whose_every_score_is_minus_infinity(native, heads, q_tokens, kv_tokens, head_dim):
+    """Keys of minus infinity in a dim where every query is one: their parts weigh nothing in the merge."""
+    gen = torch.Generator().manual_seed(kv_tokens + head_dim)
+    q = torch.randn((1, heads, q_tokens, head_dim), generator=gen)
+    k, v = (torch.randn((1, heads, kv_tokens, head_dim), generator=gen) for _ in range(2))
+    q[..., 0] = 1.0
+    k[:, :, : kv_tokens // 2, 0] = -math.inf
+    k[:, :, kv_tokens // 2 + 100:, 0] = -math.inf
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    out = native.dense_attention(q.cuda(), k.cuda(), v.cuda(), head_dim ** -0.5)
+    live = slice(kv_tokens // 2, kv_tokens // 2 + 100)
+    expected = oatt.dense_attention(np32(q), np32(k[:, :, live]), np32(v[:, :, live]))
+    assert_close(np32(out), expected, 4 * UNIT[torch.bfloat16] * 5.0, 0.0, f"{kv_tokens} keys, 100 of them live")
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("heads,tokens,exact,first_order,scale", [
     (2, 1000, 0, False, 0.125),   # centroids only: one chunk, one wave
